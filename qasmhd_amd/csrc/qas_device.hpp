@@ -39,27 +39,132 @@ template <typename T> QAS_HD T dabs(T x) { return fabs(x); }
 template <> QAS_HD float dsqrt<float>(float x) { return sqrtf(x); }
 template <> QAS_HD float dabs<float>(float x) { return fabsf(x); }
 
-// 1.0 / d for 2^-767 <= d <= 2^1022, bit-identical to the IEEE division.
+// 1.0 / d for 2^-767 <= |d| <= 2^1022, bit-identical to the IEEE division.
 // On gfx950 an FP64 division is: operand scaling (v_div_scale, twice), a
 // reciprocal estimate, two Newton steps, the quotient and its residual,
 // the corrected quotient (v_div_fmas) and the special-case fix-up
-// (v_div_fixup).  Inside that range neither operand of 1.0 / d is scaled,
-// v_div_fmas is a plain FMA and the fix-up returns its input, so the same
-// estimate, Newton steps and correction give the same bits in 7
-// instructions instead of 11.  Callers check the range.
+// (v_div_fixup).  Inside that range nothing is scaled or fixed up.  The
+// estimate is within 2^-24.3 of 1/d (measured over all leading 30 significand
+// bits), so one third-order step, r (1 + e + e^2), leaves 2^-73 before its
+// rounding; the last residual step then rounds as the division does
+// (Markstein's theorem; its one exception, a significand of all ones, is in
+// the test).  6 instructions against 7 with two Newton steps.  Callers check
+// the range.
 QAS_HD double rcp_inrange(double d)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
   double r = __builtin_amdgcn_rcp(d);
   double e = fma(-d, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-d, r, 1.0);
+  e = fma(e, e, e);
   r = fma(r, e, r);
   e = fma(-d, r, 1.0);
   return fma(e, r, r);
 #else
   return 1.0 / d;
 #endif
+}
+
+// c * a + b with c a power of two (of either sign): the product is exact, so
+// one fused operation rounds exactly as the multiply and the add do
+template <typename T>
+QAS_HD T fma2(T c, T a, T b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, double>::value) return fma(c, a, b);
+#endif
+  return c * a + b;
+}
+
+// x / N for N = 6, 24 (3 times a power of two), bit-identical to the IEEE
+// division: c = RN(1/N) is within 2^-54 of 1/N, so q = x c is within one ulp
+// of x / N, the residual x - N q is exact, and q + c (x - N q) rounds as the
+// division does; the fix-up puts signed zeros, infinities and NaN right.
+// 4 instructions against the division's 11 and its estimate.
+template <int N, typename T>
+QAS_HD T div_3p2(T x)
+{
+  static_assert(N == 6 || N == 24, "the error bound of RN(1/N) is for 3 times a power of two");
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, double>::value) {
+    constexpr double c = 1.0 / N;
+    const double q = x * c;
+    return __builtin_amdgcn_div_fixup(fma(fma(-(double)N, q, x), c, q), (double)N, x);
+  }
+#endif
+  return x / T(N);
+}
+
+// 1 / x, a / x and sqrt(x) of the point functions: FP64 on the device without
+// the IEEE sequences' operand scaling.  The scaling serves operands near the
+// ends of the exponent range; the estimate, refinement and last residual step
+// are the same, and the fix-up instruction (the class select of the root)
+// gives zeros, infinities and NaN their IEEE results.  Same bits as the
+// operators for operands and results in [2^-960, 2^1000] and for zero,
+// infinite and NaN operands.  inv 7 instructions against 11, a second quotient by
+// the same x (quot with inv_raw(x)) 4 against 11, root 13 against 18; the
+// HLLD flux forms 8 reciprocals, 4 quotients and 5 roots, which take 28 % of
+// its instructions as operators.
+template <typename T>
+QAS_HD T inv_raw(T x)
+{
+  if constexpr (std::is_same<T, double>::value) return rcp_inrange(x);
+  else return T(1.0) / x;
+}
+
+template <typename T>
+QAS_HD T inv(T x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, double>::value) return __builtin_amdgcn_div_fixup(rcp_inrange(x), x, 1.0);
+#endif
+  return T(1.0) / x;
+}
+
+// a / x with rx = inv_raw(x)
+template <typename T>
+QAS_HD T quot(T a, T x, T rx)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, double>::value) {
+    const double q = a * rx;
+    return __builtin_amdgcn_div_fixup(fma(fma(-x, q, a), rx, q), x, a);
+  }
+#endif
+  (void)rx;
+  return a / x;
+}
+
+// a / x, and 0.5 / x (an exact factor)
+template <typename T>
+QAS_HD T ratio(T a, T x)
+{
+  if constexpr (std::is_same<T, double>::value) return quot(a, x, inv_raw(x));
+  else return a / x;
+}
+
+template <typename T>
+QAS_HD T half_inv(T x)
+{
+  if constexpr (std::is_same<T, double>::value) return T(0.5) * inv(x);
+  else return T(0.5) / x;
+}
+
+template <typename T>
+QAS_HD T root(T x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, double>::value) {
+    const double r = __builtin_amdgcn_rsq(x);
+    double g = x * r, h = 0.5 * r;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0 and +inf are their own roots
+  }
+#endif
+  return dsqrt(x);
 }
 
 // ------------------------------------------------------------------ 1-D interpolation
@@ -71,8 +176,8 @@ QAS_HD void lin5(const T* f, T& fl, T& fr)
     fl = f[2];
     fr = f[2];
   } else if constexpr (ODR == 2) {
-    fl = (-f[1] + T(5.0) * f[2] + T(2.0) * f[3]) / T(6.0);
-    fr = (-f[3] + T(5.0) * f[2] + T(2.0) * f[1]) / T(6.0);
+    fl = div_3p2<6>(-f[1] + T(5.0) * f[2] + T(2.0) * f[3]);
+    fr = div_3p2<6>(-f[3] + T(5.0) * f[2] + T(2.0) * f[1]);
   } else if constexpr (ODR == 3) {
     fl = T(0.125) * (-f[1] + T(6.0) * f[2] + T(3.0) * f[3]);
     fr = T(0.125) * (-f[3] + T(6.0) * f[2] + T(3.0) * f[1]);
@@ -98,8 +203,11 @@ QAS_HD T minmod(T a, T b)
 // The weights and face values of WCNS-4 (common_interp.c:102-150) from
 // the three denominators d_k = IS_k^2 + eps; IN_RANGE takes the reciprocals
 // with rcp_inrange (FP64, the caller checked the range), else 1.0 / x.
+// Returns 8 fl and 8 fr: the face values without their factor 1/8, which is
+// exact and which lrstate folds into its coefficients.  Products with powers
+// of two go into the following add (fma2, same rounding), and 6 f = 2 (3 f).
 template <bool IN_RANGE, typename T>
-QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl, T& fr)
+QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl8, T& fr8)
 {
   auto inv = [](T x) -> T {
     if constexpr (IN_RANGE) return rcp_inrange(x);
@@ -109,12 +217,23 @@ QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl, T& fr)
   const T s1 = inv(d1);
   const T s2 = inv(d2);
   // sub-stencil values (shared by both sides)
-  const T qa = T(3.0) * f[0] - T(10.0) * f[1] + T(15.0) * f[2];
-  const T qb = -f[1] + T(6.0) * f[2] + T(3.0) * f[3];
-  const T qc = +T(3.0) * f[2] + T(6.0) * f[3] - f[4];
-  const T ra = T(3.0) * f[4] - T(10.0) * f[3] + T(15.0) * f[2];
-  const T rb = -f[3] + T(6.0) * f[2] + T(3.0) * f[1];
-  const T rc = +T(3.0) * f[2] + T(6.0) * f[1] - f[0];
+  T qa, qb, qc, ra, rb, rc;
+  if constexpr (std::is_same<T, double>::value) {
+    const T p1 = T(3.0) * f[1], p2 = T(3.0) * f[2], p3 = T(3.0) * f[3];
+    qa = T(3.0) * f[0] - T(10.0) * f[1] + T(15.0) * f[2];
+    qb = fma2(T(2.0), p2, -f[1]) + p3;
+    qc = fma2(T(2.0), p3, p2) - f[4];
+    ra = T(3.0) * f[4] - T(10.0) * f[3] + T(15.0) * f[2];
+    rb = fma2(T(2.0), p2, -f[3]) + p1;
+    rc = fma2(T(2.0), p1, p2) - f[0];
+  } else {
+    qa = T(3.0) * f[0] - T(10.0) * f[1] + T(15.0) * f[2];
+    qb = -f[1] + T(6.0) * f[2] + T(3.0) * f[3];
+    qc = +T(3.0) * f[2] + T(6.0) * f[3] - f[4];
+    ra = T(3.0) * f[4] - T(10.0) * f[3] + T(15.0) * f[2];
+    rb = -f[3] + T(6.0) * f[2] + T(3.0) * f[1];
+    rc = +T(3.0) * f[2] + T(6.0) * f[1] - f[0];
+  }
   T w0 = T(0.075) * s0;
   T w1 = T(0.650) * s1;
   T w2 = T(0.275) * s2;
@@ -122,7 +241,7 @@ QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl, T& fr)
   w0 *= den;
   w1 *= den;
   w2 = T(1.0) - w0 - w1;
-  fl = T(0.125) * (+w0 * qa + w1 * qb + w2 * qc);
+  fl8 = +w0 * qa + w1 * qb + w2 * qc;
   w0 = T(0.275) * s0;
   w1 = T(0.650) * s1;
   w2 = T(0.075) * s2;
@@ -130,12 +249,13 @@ QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl, T& fr)
   w0 *= den;
   w1 *= den;
   w2 = T(1.0) - w0 - w1;
-  fr = T(0.125) * (+w2 * ra + w1 * rb + w0 * rc);
+  fr8 = +w2 * ra + w1 * rb + w0 * rc;
 }
 
 // INRANGE: the WCNS-4 reciprocals take rcp_inrange when in range (FP64);
-// false keeps the plain division (a smaller body, for the adjoint kernels)
-template <int ODR, typename T, bool INRANGE = true>
+// false keeps the plain division (a smaller body, for the adjoint kernels).
+// S8: WCNS-4 returns 8 times the face values (exact; the caller scales).
+template <int ODR, typename T, bool INRANGE = true, bool S8 = false>
 QAS_HD void interp5(const T* f, T& fl, T& fr)
 {
   if constexpr (ODR == 1) {
@@ -168,16 +288,37 @@ QAS_HD void interp5(const T* f, T& fl, T& fr)
   } else {  // WCNS4
     const T eps = wcns_eps<T>();
     const T c13 = T(13. / 12.);
-    T a = f[0] - T(4.0) * f[1] + T(3.0) * f[2];
-    T b = f[0] - T(2.0) * f[1] + f[2];
-    const T s0 = c13 * b * b + T(0.25) * a * a;
-    a = f[1] - f[3];
-    b = f[1] - T(2.0) * f[2] + f[3];
-    const T s1 = c13 * b * b + T(0.25) * a * a;
-    a = f[4] - T(4.0) * f[3] + T(3.0) * f[2];
-    b = f[4] - T(2.0) * f[3] + f[2];
-    const T s2 = c13 * b * b + T(0.25) * a * a;
+    T s0, s1, s2;
+    if constexpr (std::is_same<T, double>::value) {
+      // the reference's expressions, powers of two fused (fma2)
+      const T p2 = T(3.0) * f[2];
+      T a = fma2(T(-4.0), f[1], f[0]) + p2;
+      T b = fma2(T(-2.0), f[1], f[0]) + f[2];
+      s0 = fma2(T(0.25), a * a, c13 * b * b);
+      a = f[1] - f[3];
+      b = fma2(T(-2.0), f[2], f[1]) + f[3];
+      s1 = fma2(T(0.25), a * a, c13 * b * b);
+      a = fma2(T(-4.0), f[3], f[4]) + p2;
+      b = fma2(T(-2.0), f[3], f[4]) + f[2];
+      s2 = fma2(T(0.25), a * a, c13 * b * b);
+    } else {
+      T a = f[0] - T(4.0) * f[1] + T(3.0) * f[2];
+      T b = f[0] - T(2.0) * f[1] + f[2];
+      s0 = c13 * b * b + T(0.25) * a * a;
+      a = f[1] - f[3];
+      b = f[1] - T(2.0) * f[2] + f[3];
+      s1 = c13 * b * b + T(0.25) * a * a;
+      a = f[4] - T(4.0) * f[3] + T(3.0) * f[2];
+      b = f[4] - T(2.0) * f[3] + f[2];
+      s2 = c13 * b * b + T(0.25) * a * a;
+    }
     const T d0 = s0 * s0 + eps, d1 = s1 * s1 + eps, d2 = s2 * s2 + eps;
+    auto fin = [&]() {
+      if constexpr (!S8) {
+        fl = T(0.125) * fl;
+        fr = T(0.125) * fr;
+      }
+    };
     if constexpr (INRANGE && std::is_same<T, double>::value) {
       // d >= eps = 1e-40 always; d <= 2^700 keeps every 1/d in
       // [2^-700, 1e40] and both weight sums in [0.65 * 2^-700, 1e40], so
@@ -185,10 +326,12 @@ QAS_HD void interp5(const T* f, T& fl, T& fr)
       // the test and takes the division)
       if ((d0 <= 0x1p700) & (d1 <= 0x1p700) & (d2 <= 0x1p700)) {
         wcns4_weights<true>(f, d0, d1, d2, fl, fr);
+        fin();
         return;
       }
     }
     wcns4_weights<false>(f, d0, d1, d2, fl, fr);
+    fin();
   }
 }
 
@@ -203,7 +346,7 @@ template <int ODR, typename T>
 QAS_HD T dfc(T fm1, T f0, T f1, T f2)
 {
   if constexpr (ODR <= 2) return (f1 - f0);
-  else return ((T(27.0) * (f1 - f0) - (f2 - fm1)) / T(24.0));
+  else return div_3p2<24>(T(27.0) * (f1 - f0) - (f2 - fm1));
 }
 
 // ------------------------------------------------------------------ characteristic reconstruction
@@ -221,12 +364,24 @@ template <int ODR, typename T, int MODE = 0, bool INRANGE = true, bool WAVEB = s
 QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int* fbc = nullptr)
 {
   const T ro0 = s[0][2], bt0 = s[4][2], bu0 = s[5][2], pr0 = s[6][2];
-  // exact-zero flags of mhd_eigen.c:575-587
+  // exact-zero flags of mhd_eigen.c:575-587: a variable whose five stencil
+  // values are all zero.  A wavefront with no zero at any cell of its own
+  // (a uniform test of 5 compares) skips the other 20.
   bool zf[5];
+#if defined(__HIP_DEVICE_COMPILE__)
+  const bool anyz = __any((s[1][2] == T(0.0)) | (s[2][2] == T(0.0)) | (s[3][2] == T(0.0)) | (s[4][2] == T(0.0)) |
+                          (s[5][2] == T(0.0))) != 0;
+#else
+  const bool anyz = true;
+#endif
 #pragma unroll
-  for (int n = 1; n <= 5; n++)
-    zf[n - 1] = (s[n][0] == T(0.0)) & (s[n][1] == T(0.0)) & (s[n][2] == T(0.0)) & (s[n][3] == T(0.0)) &
-                (s[n][4] == T(0.0));
+  for (int n = 0; n < 5; n++) zf[n] = false;
+  if (anyz) {
+#pragma unroll
+    for (int n = 1; n <= 5; n++)
+      zf[n - 1] = (s[n][0] == T(0.0)) & (s[n][1] == T(0.0)) & (s[n][2] == T(0.0)) & (s[n][3] == T(0.0)) &
+                  (s[n][4] == T(0.0));
+  }
   // branch of mhd_func.c:143 (strict >)
   const bool fast = MODE == 1 ? true : (MODE == 2 ? false : (s[0][2] * (s[1][2] * s[1][2] + s[2][2] * s[2][2] + s[3][2] * s[3][2]) > gam * s[6][2]));
   // whether the fast-only terms are formed: in WCNS-4 MODE 0 with WAVEB on
@@ -239,27 +394,29 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
   const bool anyf = MODE != 2;
 #endif
   // shared eigen quantities (mhd_eigen_mi / mhd_eigen_ae)
-  const T iro = T(1.0) / ro0;
+  const T iro = inv(ro0);
   const T cs2 = gam * pr0 * iro;
   const T ca2 = bn * bn * iro;
   const T ct2 = (bt0 * bt0 + bu0 * bu0) * iro;
   const T cb2 = cs2 + ca2 + ct2;
-  const T cf2 = T(0.5) * (cb2 + dsqrt(dabs(cb2 * cb2 - T(4.0) * cs2 * ca2)));
+  const T cf2 = T(0.5) * (cb2 + root(dabs(fma2(T(-4.0), cs2 * ca2, cb2 * cb2))));
   T rcf = T(0.0), icf2h = T(0.0), ircfh = T(0.0);
   if (MODE != 2 && anyf) {
-    const T cf = dsqrt(cf2);
+    const T cf = root(cf2);
     rcf = ro0 * cf;
   }
-  const T sro = dsqrt(ro0);
-  const T isroh = T(0.5) / sro;
-  const T icf2 = T(1.0) / cf2;
+  const T sro = root(ro0);
+  const T isroh = half_inv(sro);
+  const T icf2 = inv(cf2);
   if (MODE != 2 && anyf) {
     icf2h = T(0.5) * icf2;
-    ircfh = T(0.5) / rcf;
+    ircfh = half_inv(rcf);
   }
   const T byh = T(0.5) * bt0;
   const T bzh = T(0.5) * bu0;
 
+  // WCNS-4 in MODE 0 and FP64: face values scaled by 8 (see the back projection)
+  constexpr bool S8 = ODR == 4 && MODE == 0 && std::is_same<T, double>::value;
   T w[5], wl[7], wr[7];
   // k = 0: fast -> -rcf vn + bt0 bt + bu0 bu + pr ; Alfven/entropy -> vn
 #pragma unroll
@@ -274,11 +431,11 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
       w[m] = fast ? wf : w[m];
     }
   }
-  interp5<ODR, T, INRANGE>(w, wl[0], wr[0]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[0], wr[0]);
   // k = 1: cf2 ro - bt0 bt - bu0 bu - pr (both)
 #pragma unroll
   for (int m = 0; m < 5; m++) w[m] = cf2 * s[0][m] - bt0 * s[4][m] - bu0 * s[5][m] - s[6][m];
-  interp5<ODR, T, INRANGE>(w, wl[1], wr[1]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[1], wr[1]);
   // k = 2: fast -> rcf vn + bt0 bt + bu0 bu + pr ; A/E -> bt0 bt + bu0 bu + pr
 #pragma unroll
   for (int m = 0; m < 5; m++) {
@@ -292,22 +449,35 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
       w[m] = fast ? wf : w[m];
     }
   }
-  interp5<ODR, T, INRANGE>(w, wl[2], wr[2]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[2], wr[2]);
   // k = 3..6: Alfven pairs (both)
 #pragma unroll
   for (int m = 0; m < 5; m++) w[m] = sro * s[2][m] + s[4][m];
-  interp5<ODR, T, INRANGE>(w, wl[3], wr[3]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[3], wr[3]);
 #pragma unroll
   for (int m = 0; m < 5; m++) w[m] = sro * s[2][m] - s[4][m];
-  interp5<ODR, T, INRANGE>(w, wl[4], wr[4]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[4], wr[4]);
 #pragma unroll
   for (int m = 0; m < 5; m++) w[m] = sro * s[3][m] + s[5][m];
-  interp5<ODR, T, INRANGE>(w, wl[5], wr[5]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[5], wr[5]);
 #pragma unroll
   for (int m = 0; m < 5; m++) w[m] = sro * s[3][m] - s[5][m];
-  interp5<ODR, T, INRANGE>(w, wl[6], wr[6]);
+  interp5<ODR, T, INRANGE, S8>(w, wl[6], wr[6]);
 
-  // back projection
+  // back projection; with S8 the characteristic values are 8 times their
+  // own and the exact factor 1/8 sits in the coefficients
+  constexpr bool D = std::is_same<T, double>::value;
+  const T icf2q = S8 ? T(0.125) * icf2 : icf2;
+  const T isrohq = S8 ? T(0.125) * isroh : isroh;
+  auto q8 = [](T x) -> T {
+    if constexpr (S8) return T(0.125) * x;
+    else return x;
+  };
+  // 0.5 a - 0.5 b (FP64: the same bits as 0.5 (a - b))
+  auto half_diff = [&](T a, T b) -> T {
+    if constexpr (D) return (S8 ? T(0.0625) : T(0.5)) * (a - b);
+    else return T(0.5) * a - T(0.5) * b;
+  };
 #pragma unroll
   for (int side = 0; side < 2; side++) {
     const T* q = side ? wr : wl;
@@ -321,22 +491,22 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
       u[1] = q[0];
       u[6] = q[2] - byh * q[3] + byh * q[4] - bzh * q[5] + bzh * q[6];
     } else {
-      u[0] = icf2 * q[1] + icf2 * q[2];
-      u[1] = q[0];
-      u[6] = q[2] - byh * q[3] + byh * q[4] - bzh * q[5] + bzh * q[6];
+      u[0] = icf2q * q[1] + icf2q * q[2];
+      u[1] = q8(q[0]);
+      u[6] = q8(q[2] - byh * q[3] + byh * q[4] - bzh * q[5] + bzh * q[6]);
       if (anyf) {
-        const T rof = icf2h * q[0] + icf2 * q[1] + icf2h * q[2];
-        const T vnf = -ircfh * q[0] + ircfh * q[2];
-        const T prf = T(0.5) * q[0] + T(0.5) * q[2] - byh * q[3] + byh * q[4] - bzh * q[5] + bzh * q[6];
+        const T rof = q8(icf2h * q[0] + icf2 * q[1] + icf2h * q[2]);
+        const T vnf = q8(-ircfh * q[0] + ircfh * q[2]);
+        const T prf = q8(T(0.5) * q[0] + T(0.5) * q[2] - byh * q[3] + byh * q[4] - bzh * q[5] + bzh * q[6]);
         u[0] = fast ? rof : u[0];
         u[1] = fast ? vnf : u[1];
         u[6] = fast ? prf : u[6];
       }
     }
-    u[2] = isroh * q[3] + isroh * q[4];
-    u[3] = isroh * q[5] + isroh * q[6];
-    u[4] = T(0.5) * q[3] - T(0.5) * q[4];
-    u[5] = T(0.5) * q[5] - T(0.5) * q[6];
+    u[2] = isrohq * q[3] + isrohq * q[4];
+    u[3] = isrohq * q[5] + isrohq * q[6];
+    u[4] = half_diff(q[3], q[4]);
+    u[5] = half_diff(q[5], q[6]);
   }
 #pragma unroll
   for (int n = 0; n < 5; n++) {
@@ -379,6 +549,25 @@ QAS_HD void lr_fb(const T* p, const T* q, T bnm, T bnp, T& vl, T& vr)
 // q = (ro, vn, vt, vu, bt, bu, pr); F = (ro, mn, mt, mu, bt, bu, en)
 #define QAS_FL_EPS 1e-8
 
+// vn + b / r > 0 (r >= 0) with b / r rounded as the division rounds it.  One
+// fused operation gives the sign of vn r + b exactly, and that decides unless
+// vn is within a few roundings of -b / r (or a value is not a number), where
+// the wavefront takes the division.
+template <typename T>
+QAS_HD bool positive_sum(T vn, T b, T r)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, double>::value) {
+    const double e = fma(vn, r, b);
+    bool pos = e > 0.0;
+    const bool sure = fabs(e) > 0x1p-51 * fabs(b);
+    if (__any(!sure)) pos = sure ? pos : (vn + b / r > 0.0);
+    return pos;
+  }
+#endif
+  return vn + b / r > T(0);
+}
+
 template <typename T>
 QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, T gamma,
                                                  T dv0, T dv1, T* F)
@@ -386,53 +575,54 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   const T FL_EPS = T(QAS_FL_EPS);
   const T rol = L[0], vnl = L[1], vtl = L[2], vul = L[3], btl = L[4], bul = L[5], prl = L[6];
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
-  const T gammam1i = T(1.0) / (gamma - T(1.0));
+  const T gammam1i = inv(gamma - T(1.0));
   const T bnc2 = bnc * bnc;
   const T sgn = (bnc > T(0)) ? T(1.0) : T(-1.0);
-  const T roli = T(1.0) / rol;
-  const T pml = T(0.5) * (btl * btl + bul * bul);
-  const T ptl = prl + pml;
+  const T roli = inv(rol);
+  const T b2l = btl * btl + bul * bul;  // twice the transverse magnetic pressure
+  const T ptl = fma2(T(0.5), b2l, prl);
   const T vl2 = vnl * vnl + vtl * vtl + vul * vul;
-  const T enl = gammam1i * prl + pml + T(0.5) * rol * vl2;
+  const T enl = fma2(T(0.5), rol * vl2, fma2(T(0.5), b2l, gammam1i * prl));
   const T vbl = vtl * btl + vul * bul;
-  const T rori = T(1.0) / ror;
-  const T pmr = T(0.5) * (btr * btr + bur * bur);
-  const T ptr = prr + pmr;
+  const T rori = inv(ror);
+  const T b2r = btr * btr + bur * bur;
+  const T ptr = fma2(T(0.5), b2r, prr);
   const T vr2 = vnr * vnr + vtr * vtr + vur * vur;
-  const T enr = gammam1i * prr + pmr + T(0.5) * ror * vr2;
+  const T enr = fma2(T(0.5), ror * vr2, fma2(T(0.5), b2r, gammam1i * prr));
   const T vbr = vtr * btr + vur * bur;
   const T cl2 = gamma * prl * roli;
   const T cr2 = gamma * prr * rori;
   const T cal2 = bnc2 * roli;
   const T car2 = bnc2 * rori;
-  const T cbl2 = cl2 + cal2 + T(2.0) * pml * roli;
-  const T cbr2 = cr2 + car2 + T(2.0) * pmr * rori;
-  const T cfl2 = T(0.5) * (cbl2 + dsqrt(dabs(cbl2 * cbl2 - T(4.0) * cl2 * cal2)));
-  const T cfr2 = T(0.5) * (cbr2 + dsqrt(dabs(cbr2 * cbr2 - T(4.0) * cr2 * car2)));
-  T cmax, ccl2 = T(0), ccr2 = T(0);
+  const T cbl2 = cl2 + cal2 + b2l * roli;
+  const T cbr2 = cr2 + car2 + b2r * rori;
+  // twice the squared fast speeds
+  const T cfl2 = cbl2 + root(dabs(fma2(T(-4.0), cl2 * cal2, cbl2 * cbl2)));
+  const T cfr2 = cbr2 + root(dabs(fma2(T(-4.0), cr2 * car2, cbr2 * cbr2)));
+  T ccl2 = T(0), ccr2 = T(0);  // twice the squared speeds with |v| for the sound speed
   if (lowdiss) {
-    const T cbl2c = vl2 + cal2 + T(2.0) * pml * roli;
-    const T cbr2c = vr2 + car2 + T(2.0) * pmr * rori;
-    ccl2 = T(0.5) * (cbl2c + dsqrt(dabs(cbl2c * cbl2c - T(4.0) * vl2 * cal2)));
-    ccr2 = T(0.5) * (cbr2c + dsqrt(dabs(cbr2c * cbr2c - T(4.0) * vr2 * car2)));
-    cmax = dsqrt(tmax(cfl2, cfr2));
-  } else {
-    cmax = tmax(dsqrt(cfl2), dsqrt(cfr2));
+    const T cbl2c = vl2 + cal2 + b2l * roli;
+    const T cbr2c = vr2 + car2 + b2r * rori;
+    ccl2 = cbl2c + root(dabs(fma2(T(-4.0), vl2 * cal2, cbl2c * cbl2c)));
+    ccr2 = cbr2c + root(dabs(fma2(T(-4.0), vr2 * car2, cbr2c * cbr2c)));
   }
+  // the larger of the two fast speeds; a correctly rounded root is monotonic,
+  // so the root of the larger square is the larger root
+  const T cmax = root(T(0.5) * tmax(cfl2, cfr2));
   const T sl = tmin(T(0.0), tmin(vnl, vnr) - cmax);
   const T sr = tmax(T(0.0), tmax(vnl, vnr) + cmax);
   const T slvl = sl - vnl;
   const T srvr = sr - vnr;
   const T rslvl = rol * slvl;
   const T rsrvr = ror * srvr;
-  const T drsvi = T(1.0) / (rsrvr - rslvl);
+  const T drsvi = inv(rsrvr - rslvl);
   T vnc, ptc;
   if (lowdiss) {
-    T theta = tmin(T(1.0), (cmax - tmin(dv0, T(0.0))) / (cmax - tmin(dv1, T(0.0))));
+    T theta = tmin(T(1.0), ratio(cmax - tmin(dv0, T(0.0)), cmax - tmin(dv1, T(0.0))));
     theta *= theta;
     theta *= theta;
     vnc = (rsrvr * vnr - rslvl * vnl - theta * (ptr - ptl)) * drsvi;
-    const T mcc = tmin(T(1.0), dsqrt(tmax(ccl2, ccr2)) / cmax);
+    const T mcc = tmin(T(1.0), ratio(root(T(0.5) * tmax(ccl2, ccr2)), cmax));
     ptc = (rsrvr * ptl - rslvl * ptr + (mcc * (T(2.0) - mcc)) * rsrvr * rslvl * (vnr - vnl)) * drsvi;
   } else {
     vnc = (rsrvr * vnr - rslvl * vnl - ptr + ptl) * drsvi;
@@ -440,14 +630,16 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   }
   const T slvc = sl - vnc;
   const T srvc = sr - vnc;
-  const T ro2l = rslvl / slvc;
-  const T ro2r = rsrvr / srvc;
+  const T slvci = inv_raw(slvc);
+  const T srvci = inv_raw(srvc);
+  const T ro2l = quot(rslvl, slvc, slvci);
+  const T ro2r = quot(rsrvr, srvc, srvci);
   const T rhdl = rslvl * slvc - bnc2;
   const T rhdr = rsrvr * srvc - bnc2;
   T vt2l = vtl, vu2l = vul, bt2l = btl, bu2l = bul;
   T vt2r = vtr, vu2r = vur, bt2r = btr, bu2r = bur;
   if (dabs(rhdl) > FL_EPS) {
-    const T rhdli = T(1.0) / rhdl;
+    const T rhdli = inv(rhdl);
     const T rhnvl = (vnl - vnc) * bnc;
     const T rhnbl = rslvl * slvl - bnc2;
     vt2l = vtl + rhnvl * rhdli * btl;
@@ -456,7 +648,7 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
     bu2l = rhnbl * rhdli * bul;
   }
   if (dabs(rhdr) > FL_EPS) {
-    const T rhdri = T(1.0) / rhdr;
+    const T rhdri = inv(rhdr);
     const T rhnvr = (vnr - vnc) * bnc;
     const T rhnbr = rsrvr * srvr - bnc2;
     vt2r = vtr + rhnvr * rhdri * btr;
@@ -466,23 +658,23 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   }
   const T vb2l = vt2l * bt2l + vu2l * bu2l;
   const T vb2r = vt2r * bt2r + vu2r * bu2r;
-  const T en2l = (slvl * enl - ptl * vnl + ptc * vnc + bnc * (vbl - vb2l)) / slvc;
-  const T en2r = (srvr * enr - ptr * vnr + ptc * vnc + bnc * (vbr - vb2r)) / srvc;
-  const T rro2l = dsqrt(ro2l);
-  const T rro2r = dsqrt(ro2r);
-  const T rro2i = T(1.0) / (rro2r + rro2l);
-  const T vt3m = (rro2r * vt2r + rro2l * vt2l + (bt2r - bt2l) * sgn) * rro2i;
-  const T vu3m = (rro2r * vu2r + rro2l * vu2l + (bu2r - bu2l) * sgn) * rro2i;
-  const T bt3m = (rro2l * bt2r + rro2r * bt2l + rro2r * rro2l * (vt2r - vt2l) * sgn) * rro2i;
-  const T bu3m = (rro2l * bu2r + rro2r * bu2l + rro2r * rro2l * (vu2r - vu2l) * sgn) * rro2i;
+  const T en2l = quot(slvl * enl - ptl * vnl + ptc * vnc + bnc * (vbl - vb2l), slvc, slvci);
+  const T en2r = quot(srvr * enr - ptr * vnr + ptc * vnc + bnc * (vbr - vb2r), srvc, srvci);
+  const T rro2l = root(ro2l);
+  const T rro2r = root(ro2r);
+  const T rro2i = inv(rro2r + rro2l);
+  const T vt3m = fma2(sgn, bt2r - bt2l, rro2r * vt2r + rro2l * vt2l) * rro2i;
+  const T vu3m = fma2(sgn, bu2r - bu2l, rro2r * vu2r + rro2l * vu2l) * rro2i;
+  const T bt3m = fma2(sgn, rro2r * rro2l * (vt2r - vt2l), rro2l * bt2r + rro2r * bt2l) * rro2i;
+  const T bu3m = fma2(sgn, rro2r * rro2l * (vu2r - vu2l), rro2l * bu2r + rro2r * bu2l) * rro2i;
   const T vb3m = vt3m * bt3m + vu3m * bu3m;
-  const T en3l = en2l - rro2l * (vb2l - vb3m) * sgn;
-  const T en3r = en2r + rro2r * (vb2r - vb3m) * sgn;
+  const T en3l = fma2(-sgn, rro2l * (vb2l - vb3m), en2l);
+  const T en3r = fma2(sgn, rro2r * (vb2r - vb3m), en2r);
   const T hl = (vnc > T(0)) ? T(1.0) : T(0.0);
   const T hr = T(1.0) - hl;
-  const T h2l = (vnc - dabs(bnc) / rro2l > T(0)) ? T(1.0) : T(0.0);
+  const T h2l = positive_sum(vnc, -dabs(bnc), rro2l) ? T(1.0) : T(0.0);
   const T h3l = (T(1.0) - h2l) * hl;
-  const T h2r = (vnc + dabs(bnc) / rro2r > T(0)) ? T(0.0) : T(1.0);
+  const T h2r = positive_sum(vnc, dabs(bnc), rro2r) ? T(0.0) : T(1.0);
   const T h3r = (T(1.0) - h2r) * hr;
   const T rou = ro2l * hl + ro2r * hr;
   const T vtu = vt2l * h2l + vt3m * (h3l + h3r) + vt2r * h2r;
@@ -491,7 +683,7 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   const T buu = bu2l * h2l + bu3m * (h3l + h3r) + bu2r * h2r;
   const T enu = en2l * h2l + en3l * h3l + en3r * h3r + en2r * h2r;
   F[0] = rou * vnc;
-  F[1] = rou * vnc * vnc + ptc - bnc2 * T(0.5);
+  F[1] = fma2(T(-0.5), bnc2, rou * vnc * vnc + ptc);
   F[2] = rou * vtu * vnc - bnc * btu;
   F[3] = rou * vuu * vnc - bnc * buu;
   F[4] = btu * vnc - bnc * vtu;
@@ -505,17 +697,17 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T FL_EPS = T(QAS_FL_EPS);
   const T rol = L[0], vnl = L[1], vtl = L[2], vul = L[3], btl = L[4], bul = L[5], prl = L[6];
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
-  const T gammam1i = T(1.0) / (gamma - T(1.0));
+  const T gammam1i = inv(gamma - T(1.0));
   const T bnc2 = bnc * bnc;
   const T sgn = (bnc > T(0)) ? T(1.0) : T(-1.0);
   const T bnca = sgn * bnc;
-  const T roli = T(1.0) / rol;
+  const T roli = inv(rol);
   const T vl2 = vnl * vnl + vtl * vtl + vul * vul;
   const T pml = T(0.5) * (btl * btl + bul * bul);
   const T ptl = prl + pml;
   const T enl = gammam1i * prl + pml + T(0.5) * rol * vl2;
   const T hnl = (enl + ptl) * roli;
-  const T rori = T(1.0) / ror;
+  const T rori = inv(ror);
   const T vr2 = vnr * vnr + vtr * vtr + vur * vur;
   const T pmr = T(0.5) * (btr * btr + bur * bur);
   const T ptr = prr + pmr;
@@ -527,22 +719,22 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T car2 = bnc2 * rori;
   T cbl2 = cl2 + cal2 + T(2.0) * pml * roli;
   T cbr2 = cr2 + car2 + T(2.0) * pmr * rori;
-  const T cfl2 = T(0.5) * (cbl2 + dsqrt(dabs(cbl2 * cbl2 - T(4.0) * cl2 * cal2)));
-  const T cfr2 = T(0.5) * (cbr2 + dsqrt(dabs(cbr2 * cbr2 - T(4.0) * cr2 * car2)));
+  const T cfl2 = T(0.5) * (cbl2 + root(dabs(cbl2 * cbl2 - T(4.0) * cl2 * cal2)));
+  const T cfr2 = T(0.5) * (cbr2 + root(dabs(cbr2 * cbr2 - T(4.0) * cr2 * car2)));
   cbl2 = vl2 + cal2 + T(2.0) * pml * roli;
   cbr2 = vr2 + car2 + T(2.0) * pmr * rori;
-  const T ccl2 = T(0.5) * (cbl2 + dsqrt(dabs(cbl2 * cbl2 - T(4.0) * vl2 * cal2)));
-  const T ccr2 = T(0.5) * (cbr2 + dsqrt(dabs(cbr2 * cbr2 - T(4.0) * vr2 * car2)));
-  const T cmax = dsqrt(tmax(cfl2, cfr2));
+  const T ccl2 = T(0.5) * (cbl2 + root(dabs(cbl2 * cbl2 - T(4.0) * vl2 * cal2)));
+  const T ccr2 = T(0.5) * (cbr2 + root(dabs(cbr2 * cbr2 - T(4.0) * vr2 * car2)));
+  const T cmax = root(tmax(cfl2, cfr2));
   const T cfn = cmax;
-  const T cfni = T(1.0) / cfn;
+  const T cfni = inv(cfn);
   const T sl = tmin(T(0.0), tmin(vnl, vnr) - cmax);
   const T sr = tmax(T(0.0), tmax(vnl, vnr) + cmax);
   const T mal = vnl * cfni;
   const T mar = vnr * cfni;
   const T snl = (mal > T(0)) ? T(1.0) : T(-1.0);
   const T snr = (mar > T(0)) ? T(1.0) : T(-1.0);
-  T theta = tmin(T(1.0), (cfn - tmin(dv0, T(0.0))) / (cfn - tmin(dv1, T(0.0))));
+  T theta = tmin(T(1.0), ratio(cfn - tmin(dv0, T(0.0)), cfn - tmin(dv1, T(0.0))));
   theta *= theta;
   theta *= theta;
   const T alpha = T(0.1875);
@@ -568,7 +760,7 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   }
   const T mnc = ffl + ffr;
   T mflux = mnc * cfn;
-  mflux -= tmax(T(1.0) - dabs(mnc), T(0.0)) * theta * cfni * (ptr - ptl) / (rol + ror);
+  mflux -= ratio(tmax(T(1.0) - dabs(mnc), T(0.0)) * theta * cfni * (ptr - ptl), rol + ror);
   const T dir = (mflux > T(0)) ? T(1.0) : T(-1.0);
   const T dirl = T(0.5) * (T(1.0) + dir);
   const T dirr = T(1.0) - dirl;
@@ -576,31 +768,31 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T mfl = mflux * dirl;
   const T mfr = mflux - mfl;
   T ptot = bfl * ptl + bfr * ptr;
-  const T cfmod = dsqrt(tmax(ccl2, ccr2));
+  const T cfmod = root(tmax(ccl2, ccr2));
   ptot -= T(0.25) * bfl * bfr * (rol + ror) * cfmod * (vnr - vnl);
   ptot -= T(0.5) * (T(1.0) - cfmod * cfni) * (bfl + bfr - T(1.0)) * (ptl + ptr);
   const T slvl = sl - vnl;
   const T srvr = sr - vnr;
   const T snc = dirl * sl + dirr * sr;
   const T vndnm = mflux + dirl * rol * slvl + dirr * ror * srvr;
-  const T vnc = ((dabs(vndnm) > FL_EPS) && (snc != T(0))) ? (mflux * snc / vndnm) : (dirl * vnl + dirr * vnr);
+  const T vnc = ((dabs(vndnm) > FL_EPS) && (snc != T(0))) ? ratio(mflux * snc, vndnm) : (dirl * vnl + dirr * vnr);
   const T slvc = sl - vnc;
   const T srvc = sr - vnc;
-  const T slvci = T(1.0) / slvc;
-  const T srvci = T(1.0) / srvc;
+  const T slvci = inv(slvc);
+  const T srvci = inv(srvc);
   const T rhdl = rol * slvl * slvc - bnc2;
   const T rhdr = ror * srvr * srvc - bnc2;
   T dvtl = T(0.0), dvul = T(0.0), dbtl = T(0.0), dbul = T(0.0);
   T dvtr = T(0.0), dvur = T(0.0), dbtr = T(0.0), dbur = T(0.0);
   if (dabs(rhdl) > FL_EPS) {
-    const T q = (vnc - vnl) / rhdl;
+    const T q = ratio(vnc - vnl, rhdl);
     dvtl = -bnc * btl * q;
     dvul = -bnc * bul * q;
     dbtl = bnc2 * btl * q * slvci;
     dbul = bnc2 * bul * q * slvci;
   }
   if (dabs(rhdr) > FL_EPS) {
-    const T q = (vnc - vnr) / rhdr;
+    const T q = ratio(vnc - vnr, rhdr);
     dvtr = -bnc * btr * q;
     dvur = -bnc * bur * q;
     dbtr = bnc2 * btr * q * srvci;
@@ -609,24 +801,24 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T cmpl = slvl * slvci;
   const T cmpr = srvr * srvci;
   const T ro2l = rol * cmpl;
-  const T srol = dsqrt(ro2l);
+  const T srol = root(ro2l);
   const T vt2l = dvtl + vtl;
   const T vu2l = dvul + vul;
   const T bt2l = dbtl + btl * cmpl;
   const T bu2l = dbul + bul * cmpl;
   const T ro2r = ror * cmpr;
-  const T sror = dsqrt(ro2r);
+  const T sror = root(ro2r);
   const T vt2r = dvtr + vtr;
   const T vu2r = dvur + vur;
   const T bt2r = dbtr + btr * cmpr;
   const T bu2r = dbur + bur * cmpr;
-  const T sroi = T(1.0) / (srol + sror);
+  const T sroi = inv(srol + sror);
   const T srollri = srol * sroi;
   const T srorlri = sror * sroi;
   const T bnflb = sgn * tmin(tmax(T(0.0), srollri * (bnca + sror * vnc)), bnca);
   const T bnfrb = sgn * tmin(tmax(T(0.0), srorlri * (bnca - srol * vnc)), bnca);
-  const T bnflv = sgn * tmin(tmax(T(0.0), srorlri * (bnca + mflux / sror)), bnca);
-  const T bnfrv = sgn * tmin(tmax(T(0.0), srollri * (bnca - mflux / srol)), bnca);
+  const T bnflv = sgn * tmin(tmax(T(0.0), srorlri * (bnca + ratio(mflux, sror))), bnca);
+  const T bnfrv = sgn * tmin(tmax(T(0.0), srollri * (bnca - ratio(mflux, srol))), bnca);
   const T bnsrv = tmax(bnca - dir * vnc * (dirl * srol + dirr * sror), T(0.0));
   const T ccb = sroi * bnsrv;
   const T ccv = srol * sror * ccb;
@@ -649,8 +841,9 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   rv2b2 *= rv2b2;
   T vb3 = T(0.0);
   if (rv2b2 > FL_EPS * FL_EPS) {
-    vb3 = (+(fmt * vnc + fbt * bnc) * (fmt * bnc + fbt * mflux) + (fmu * vnc + fbu * bnc) * (fmu * bnc + fbu * mflux)) /
-          rv2b2;
+    vb3 = ratio(+(fmt * vnc + fbt * bnc) * (fmt * bnc + fbt * mflux) +
+                    (fmu * vnc + fbu * bnc) * (fmu * bnc + fbu * mflux),
+                rv2b2);
   }
   const T bnvb = sgn * (bnca * (snc * vb2 - vnc * vb1) * (dirl * slvci + dirr * srvci) + bnsrv * (vb3 - vb2));
   F[0] = mflux;
@@ -670,16 +863,16 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
   const T gammam1 = gamma - T(1.0);
   const T gammam2 = gamma - T(2.0);
-  const T gammam1i = T(1.0) / gammam1;
-  const T roli = T(1.0) / rol;
-  const T rori = T(1.0) / ror;
-  const T rrol = dsqrt(rol);
-  const T rror = dsqrt(ror);
-  const T rroi = T(1.0) / (rrol + rror);
+  const T gammam1i = inv(gammam1);
+  const T roli = inv(rol);
+  const T rori = inv(ror);
+  const T rrol = root(rol);
+  const T rror = root(ror);
+  const T rroi = inv(rrol + rror);
   const T robar = rrol * rror;
-  const T robari = T(1.0) / robar;
-  const T rrobar = dsqrt(robar);
-  const T rrobai = dsqrt(robari);
+  const T robari = inv(robar);
+  const T rrobar = root(robar);
+  const T rrobai = root(robari);
   const T vnbar = (rrol * vnl + rror * vnr) * rroi;
   const T vtbar = (rrol * vtl + rror * vtr) * rroi;
   const T vubar = (rrol * vul + rror * vur) * rroi;
@@ -701,28 +894,28 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T a2 = (gammam1 * (+hbar - v2b - db2) - gammam2 * bb2 * robari);
   const T ca2 = bnbar * bnbar * robari;
   const T cb2 = (btbar * btbar + bubar * bubar) * robari;
-  const T cf2 = T(0.5) * (a2 + dsqrt(cb2 * (a2 + c2 + ca2) + (c2 - ca2) * (c2 - ca2)));
-  const T cs2 = c2 * ca2 / cf2;
-  const T cf = dsqrt(cf2);
-  const T cs = dsqrt(cs2);
-  const T ca = dsqrt(ca2);
-  const T c = dsqrt(c2);
-  const T cfi = T(1.0) / cf;
+  const T cf2 = T(0.5) * (a2 + root(cb2 * (a2 + c2 + ca2) + (c2 - ca2) * (c2 - ca2)));
+  const T cs2 = ratio(c2 * ca2, cf2);
+  const T cf = root(cf2);
+  const T cs = root(cs2);
+  const T ca = root(ca2);
+  const T c = root(c2);
+  const T cfi = inv(cf);
   const T sgr1 = btbar * btbar + bubar * bubar - FL_EPS;
   const T sf11 = (sgr1 > T(0)) ? T(1.0) : T(0.0);
   const T sf21 = T(1.0) - sf11;
-  const T beti = T(1.0) / dsqrt(btbar * btbar + bubar * bubar + sf21);
-  const T bett = sf11 * btbar * beti + sf21 * dsqrt(T(0.5));
-  const T betu = sf11 * bubar * beti + sf21 * dsqrt(T(0.5));
+  const T beti = inv(root(btbar * btbar + bubar * bubar + sf21));
+  const T bett = sf11 * btbar * beti + sf21 * root(T(0.5));
+  const T betu = sf11 * bubar * beti + sf21 * root(T(0.5));
   const T sgr2 = (btbar * btbar + bubar * bubar) * robari + dabs(ca2 - c2) - FL_EPS;
   const T sf12 = (sgr2 > T(0)) ? T(1.0) : T(0.0);
   const T sf22 = T(1.0) - sf12;
   const T cfca = tmax(T(0.0), cf2 - ca2);
   const T cfcs = tmax(T(0.0), cf2 - cs2);
   const T cfa = tmax(T(0.0), cf2 - c2);
-  const T alpi = T(1.0) / dsqrt(cfcs + sf22);
-  const T alpf = sf12 * dsqrt(cfca) * alpi + sf22;
-  const T alps = sf12 * dsqrt(cfa) * alpi;
+  const T alpi = inv(root(cfcs + sf22));
+  const T alpf = sf12 * root(cfca) * alpi + sf22;
+  const T alps = sf12 * root(cfa) * alpi;
   const T eeps = T(0.0);
   const T evpf = tmax(dabs(vnbar + cf), eeps);
   const T evmf = tmax(dabs(vnbar - cf), eeps);
@@ -751,8 +944,8 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T q12 = alps * cs;
   const T q21 = -alps * ca * sgn;
   const T q22 = alpf * c * sgn;
-  const T detpi = T(1.0) / (p11 * p22 - p12 * p21);
-  const T detqi = T(1.0) / (q11 * q22 - q12 * q21);
+  const T detpi = inv(p11 * p22 - p12 * p21);
+  const T detqi = inv(q11 * q22 - q12 * q21);
   const T wvpf = T(0.5) * ((p22 * t1 - p12 * t2) * detpi + (q22 * s1 - q12 * s2) * detqi);
   const T wvmf = T(0.5) * ((p22 * t1 - p12 * t2) * detpi - (q22 * s1 - q12 * s2) * detqi);
   const T wvps = T(0.5) * ((-p21 * t1 + p11 * t2) * detpi + (-q21 * s1 + q11 * s2) * detqi);

@@ -306,7 +306,7 @@ __global__ __launch_bounds__(256, 2) void k_sweep3d_t(StagePtrs p, Geo g, BcFlag
 // One wavefront per 60-face segment of an x line; runs after the z and y
 // sweeps and applies the RK stage sum.
 template <int DIR, int RMN, int ODR, typename T, int FMA = 0>
-__global__ __launch_bounds__(256) void k_sweep3d(StagePtrs p, Geo g, BcFlags bc, double gam, int nseg)
+__global__ __launch_bounds__(256, sizeof(T) == 8 && RMN == 1 ? 3 : 1) void k_sweep3d(StagePtrs p, Geo g, BcFlags bc, double gam, int nseg)
 {
   constexpr int TA = (DIR + 1) % 3;  // first transverse axis (t)
   constexpr int TB = (DIR + 2) % 3;  // second transverse axis (u)

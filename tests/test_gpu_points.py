@@ -108,3 +108,51 @@ def test_flux(pts, rmn, g):
 def test_cuct(pts):
     print("case: cuct", flush=True)
     assert np.array_equal(pts.cuct(U["cuct_c"], U["cuct_b"]), U["cuct"])
+
+
+def test_df_across_magnitudes(pts, oracle):
+    """The 4th-order difference's division by 24 (a product with the rounded
+    1/24 and one exact residual step) on differences from 1e-280 to 1e280,
+    signed zeros, infinities and NaN: the bits of the oracle's division."""
+    print("case: df over magnitudes", flush=True)
+    rng = np.random.default_rng(31)
+    f4 = rng.standard_normal((281 * 512, 4)) * np.repeat(10.0 ** np.arange(-280, 281, 2), 512)[:, None]
+    ints = rng.integers(-200, 200, (4096, 4)).astype(float)     # exact quotients and ties among them
+    odd = np.array([[0.0, 0.0, 0.0, 0.0], [0.0, -0.0, -0.0, 0.0], [1.0, 2.0, 2.0, 1.0], [np.inf, 1.0, 2.0, 3.0],
+                    [1.0, np.inf, 1.0, 1.0], [np.nan, 1.0, 1.0, 1.0]])
+    f4 = np.concatenate([f4, ints, odd])
+    out, ref = pts.f4(1, 4, f4), oracle.df(4, f4)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(out), nan)
+    assert np.array_equal(out[~nan].view(np.int64), ref[~nan].view(np.int64))
+
+
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+def test_flux_across_magnitudes(pts, oracle, rmn):
+    """The fluxes' reciprocals, quotients and roots without operand scaling,
+    on states whose density, speed and pressure run over 1e-40 .. 1e40 (all
+    intermediate values inside 2^-960 .. 2^960), on states at rest, without
+    field, with equal sides, and with the contact at exactly the speed of a
+    rotational wave: the oracle's values, NaN where it has NaN."""
+    print("case: flux over magnitudes, rmn", rmn, flush=True)
+    rng = np.random.default_rng(40 + rmn)
+    n = 40000
+    q = rng.uniform(0.5, 2.0, (2, n, 7)) * np.where(np.arange(7) % 6 == 0, 1.0, rng.choice([-1.0, 1.0], (2, n, 7)))
+    bn = rng.uniform(-2.0, 2.0, n)
+    dv = rng.uniform(-0.2, 0.2, (n, 2))
+    a, b = 10.0 ** rng.uniform(-40, 40, n), 10.0 ** rng.uniform(-25, 25, n)
+    scale = np.stack([a, b, b, b, np.sqrt(a) * b, np.sqrt(a) * b, a * b * b], axis=1)
+    scale[:n // 4] = 1.0
+    q = q * scale
+    bn, dv = bn * scale[:, 4], dv * scale[:, 1:2]
+    k = n // 64                      # special states, at scale 1
+    q[1, :k] = q[0, :k]              # equal sides
+    q[:, k:2 * k, 1:4] = 0.0         # at rest
+    q[:, 2 * k:3 * k, 4:6] = 0.0     # no field
+    bn[2 * k:3 * k] = 0.0
+    q[1, 3 * k:4 * k] = q[0, 3 * k:4 * k]   # equal sides with v_n = |B_n| / sqrt(ro): ro = 1, 4
+    q[:, 3 * k:4 * k, 0] = rng.choice([1.0, 4.0], k)
+    bn[3 * k:4 * k] = rng.integers(1, 16, k) / 8.0
+    q[:, 3 * k:4 * k, 1] = bn[3 * k:4 * k] / np.sqrt(q[0, 3 * k:4 * k, 0]) * rng.choice([-1.0, 1.0], k)
+    out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
+    assert _eq_nan(out, ref)
