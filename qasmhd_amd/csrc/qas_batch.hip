@@ -238,12 +238,11 @@ static int fill_table(qas_batch* b)
     B.hcap = c->hist_cap;
     B.nghost = (long long)g.nx * g.ny - (long long)(g.nx - 2 * NG) * (g.ny - 2 * NG);
     B.cfl_dr = c->s.cfl * ((g.dx >= g.dy) ? g.dy : g.dx);
-    B.nsx = (g.nx - 5 + SEG - 1) / SEG;
-    B.nsy = (g.ny - 5 + SEG - 1) / SEG;
+    B.bundle = ysweep2d_bundle(g, true);
     const long long ninter = (long long)(g.nx - 2 * NG) * (g.ny - 2 * NG);
     B.cflblocks = std::min(cdiv(ninter, 256), CFL_MAX_BLOCKS);
-    const int cnt[BK_COUNT] = {cdiv((long long)B.nsx * g.ny * WAVE, (long long)WAVE * b->xwpb),
-                               ((g.nx + YC - 1) / YC) * B.nsy,
+    const int cnt[BK_COUNT] = {(int)xsweep2d_blocks(g, b->xwpb),
+                               ysweep2d_blocks(g, B.bundle),
                                cdiv((long long)(g.nx - 5) * ((g.ny - 5 + 1) / 2), b->ewb),
                                cdiv((long long)(g.nx - 7) * (g.ny - 7), b->ewb),
                                cdiv(B.nghost * 8, 256),
@@ -285,8 +284,8 @@ static hipError_t launch_stage_all(qas_batch* b, int rk, const BatchInst* tbl = 
   const unsigned eb = (unsigned)b->ewb, xb = (unsigned)(WAVE * b->xwpb);
   hipLaunchKernelGGL(b->sy, (unsigned)b->nblk[BK_SY], 256, 0, st, StagePtrs{}, Geo{}, BcFlags{}, b->s.gam, 0, I,
                      boff(b, BK_SY), n, rk);
-  hipLaunchKernelGGL(b->sx, (unsigned)b->nblk[BK_SX], xb, 0, st, StagePtrs{}, Geo{}, BcFlags{}, b->s.gam, 0, I,
-                     boff(b, BK_SX), n, rk);
+  hipLaunchKernelGGL(b->sx, (unsigned)b->nblk[BK_SX], xb, xsweep2d_lds(b->xwpb, b->s.precision == 1), st,
+                     StagePtrs{}, Geo{}, BcFlags{}, b->s.gam, 0, I, boff(b, BK_SX), n, rk);
   if (faces_only) return hipGetLastError();
   hipLaunchKernelGGL(b->emf, (unsigned)b->nblk[BK_EMF], eb, 0, st, I, boff(b, BK_EMF), n, rk, b->s.ctw);
   hipLaunchKernelGGL(b->ct, (unsigned)b->nblk[BK_CT], eb, 0, st, I, boff(b, BK_CT), n, rk);

@@ -26,9 +26,8 @@ struct BatchInst {
   long long hcap;
   long long nghost;  // ghost cells per array
   double cfl_dr;     // cfl * min(dx, dy)
-  int nsx, nsy;      // sweep segments along x and y
   int cflblocks;     // blocks of this instance's CFL reduction
-  int pad;
+  int bundle;        // column groups per bundle of the y sweep's tiles
 };
 
 // instance owning block b: off[0..n] ascending, off[0] = 0, off[n] = grid
@@ -44,12 +43,18 @@ __device__ __forceinline__ int batch_find(const int* off, int n, int b)
 }
 
 typedef void (*batch_fn)(const BatchInst*, const int*, int, int, double);
-// the 2D sweeps: (stage descriptor, geometry, boundary flags, gam, segments)
-// for one domain, (instance table, block offsets, instances, stage) for a batch
+// the 2D sweeps: (stage descriptor, geometry, boundary flags, gam, bundle of
+// the y tiles) for one domain, (instance table, block offsets, instances,
+// stage) for a batch
 typedef void (*xsweep2d_fn)(StagePtrs, Geo, BcFlags, double, int, const BatchInst*, const int*, int, int);
 
 // kernel tables (instantiated in qas_kernels2d.hip for FP64, in
 // qas_mixed.hip for the mixed path and in qas_fma64.hip for contracted FP64)
+// workgroups of the two (x: wpb wavefronts each; its LDS bytes)
+inline int ysweep2d_bundle(const Geo& g, bool batch) { return line_bundle((g.nx + 3) / 4, g.ny, batch ? 1 << 20 : 1); }
+inline int ysweep2d_blocks(const Geo& g, int bundle) { return line_tiles((g.nx + 3) / 4, g.ny, bundle); }
+inline long long xsweep2d_blocks(const Geo& g, int wpb) { return (g.nd + WAVE * wpb - HALO - 1) / (WAVE * wpb - HALO); }
+unsigned xsweep2d_lds(int wpb, bool f32);
 xsweep2d_fn pick_ysweep2d(int rmn, int odr, bool batch);
 xsweep2d_fn pick_ysweep2d_f32(int rmn, int odr, bool batch);
 xsweep2d_fn pick_xsweep2d(int rmn, int odr, bool batch);

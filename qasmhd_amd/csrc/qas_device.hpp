@@ -350,7 +350,9 @@ QAS_HD T dfc(T fm1, T f0, T f1, T f2)
 }
 
 // ------------------------------------------------------------------ characteristic reconstruction
-// s[k][m]: k = (ro, vn, vt, vu, bt, bu, pr), m = stencil i-2..i+2.
+// s(k, m): k = (ro, vn, vt, vu, bt, bu, pr), m = 0..4 for cells i-2..i+2;
+// s.again() between the characteristic fields lets a stencil in LDS be read
+// again instead of being held in registers.
 // bn: cell-centred normal B.  vl: face i+1/2 (left state), vr: face i-1/2.
 // MODE 0: both projections formed, selected per lane (the kernels); in the
 // WCNS-4 instances with WAVEB (FP64, and the FP32 LHLLD / MLAU y sweeps)
@@ -360,17 +362,17 @@ QAS_HD T dfc(T fm1, T f0, T f1, T f2)
 // MODE 1 / 2: only the fast/Alfven resp. Alfven/entropy projection is
 // evaluated (used by the flop model to count one branch).  fbc, when given,
 // receives the positivity-fallback flags (1: left state, 2: right state).
-template <int ODR, typename T, int MODE = 0, bool INRANGE = true, bool WAVEB = std::is_same<T, double>::value>
-QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int* fbc = nullptr)
+template <int ODR, typename T, int MODE, bool INRANGE, bool WAVEB, typename S>
+QAS_HD void lrstate_of(const S& s, T bn, T gam, T (&vl)[7], T (&vr)[7], int* fbc = nullptr)
 {
-  const T ro0 = s[0][2], bt0 = s[4][2], bu0 = s[5][2], pr0 = s[6][2];
+  const T ro0 = s(0, 2), bt0 = s(4, 2), bu0 = s(5, 2), pr0 = s(6, 2);
   // exact-zero flags of mhd_eigen.c:575-587: a variable whose five stencil
   // values are all zero.  A wavefront with no zero at any cell of its own
   // (a uniform test of 5 compares) skips the other 20.
   bool zf[5];
 #if defined(__HIP_DEVICE_COMPILE__)
-  const bool anyz = __any((s[1][2] == T(0.0)) | (s[2][2] == T(0.0)) | (s[3][2] == T(0.0)) | (s[4][2] == T(0.0)) |
-                          (s[5][2] == T(0.0))) != 0;
+  const bool anyz = __any((s(1, 2) == T(0.0)) | (s(2, 2) == T(0.0)) | (s(3, 2) == T(0.0)) | (s(4, 2) == T(0.0)) |
+                          (s(5, 2) == T(0.0))) != 0;
 #else
   const bool anyz = true;
 #endif
@@ -379,11 +381,11 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
   if (anyz) {
 #pragma unroll
     for (int n = 1; n <= 5; n++)
-      zf[n - 1] = (s[n][0] == T(0.0)) & (s[n][1] == T(0.0)) & (s[n][2] == T(0.0)) & (s[n][3] == T(0.0)) &
-                  (s[n][4] == T(0.0));
+      zf[n - 1] = (s(n, 0) == T(0.0)) & (s(n, 1) == T(0.0)) & (s(n, 2) == T(0.0)) & (s(n, 3) == T(0.0)) &
+                  (s(n, 4) == T(0.0));
   }
   // branch of mhd_func.c:143 (strict >)
-  const bool fast = MODE == 1 ? true : (MODE == 2 ? false : (s[0][2] * (s[1][2] * s[1][2] + s[2][2] * s[2][2] + s[3][2] * s[3][2]) > gam * s[6][2]));
+  const bool fast = MODE == 1 ? true : (MODE == 2 ? false : (s(0, 2) * (s(1, 2) * s(1, 2) + s(2, 2) * s(2, 2) + s(3, 2) * s(3, 2)) > gam * s(6, 2)));
   // whether the fast-only terms are formed: in WCNS-4 MODE 0 with WAVEB on
   // the device, when any lane of the wavefront takes the fast branch (a
   // uniform value)
@@ -421,48 +423,52 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
   // k = 0: fast -> -rcf vn + bt0 bt + bu0 bu + pr ; Alfven/entropy -> vn
 #pragma unroll
   for (int m = 0; m < 5; m++) {
-    if (MODE == 1) w[m] = -rcf * s[1][m] + bt0 * s[4][m] + bu0 * s[5][m] + s[6][m];
-    else w[m] = s[1][m];
+    if (MODE == 1) w[m] = -rcf * s(1, m) + bt0 * s(4, m) + bu0 * s(5, m) + s(6, m);
+    else w[m] = s(1, m);
   }
   if (MODE == 0 && anyf) {
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-      const T wf = -rcf * s[1][m] + bt0 * s[4][m] + bu0 * s[5][m] + s[6][m];
+      const T wf = -rcf * s(1, m) + bt0 * s(4, m) + bu0 * s(5, m) + s(6, m);
       w[m] = fast ? wf : w[m];
     }
   }
   interp5<ODR, T, INRANGE, S8>(w, wl[0], wr[0]);
+  s.again();
   // k = 1: cf2 ro - bt0 bt - bu0 bu - pr (both)
 #pragma unroll
-  for (int m = 0; m < 5; m++) w[m] = cf2 * s[0][m] - bt0 * s[4][m] - bu0 * s[5][m] - s[6][m];
+  for (int m = 0; m < 5; m++) w[m] = cf2 * s(0, m) - bt0 * s(4, m) - bu0 * s(5, m) - s(6, m);
   interp5<ODR, T, INRANGE, S8>(w, wl[1], wr[1]);
   // k = 2: fast -> rcf vn + bt0 bt + bu0 bu + pr ; A/E -> bt0 bt + bu0 bu + pr
 #pragma unroll
   for (int m = 0; m < 5; m++) {
-    if (MODE == 1) w[m] = rcf * s[1][m] + bt0 * s[4][m] + bu0 * s[5][m] + s[6][m];
-    else w[m] = bt0 * s[4][m] + bu0 * s[5][m] + s[6][m];
+    if (MODE == 1) w[m] = rcf * s(1, m) + bt0 * s(4, m) + bu0 * s(5, m) + s(6, m);
+    else w[m] = bt0 * s(4, m) + bu0 * s(5, m) + s(6, m);
   }
   if (MODE == 0 && anyf) {
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-      const T wf = rcf * s[1][m] + bt0 * s[4][m] + bu0 * s[5][m] + s[6][m];
+      const T wf = rcf * s(1, m) + bt0 * s(4, m) + bu0 * s(5, m) + s(6, m);
       w[m] = fast ? wf : w[m];
     }
   }
   interp5<ODR, T, INRANGE, S8>(w, wl[2], wr[2]);
+  s.again();
   // k = 3..6: Alfven pairs (both)
 #pragma unroll
-  for (int m = 0; m < 5; m++) w[m] = sro * s[2][m] + s[4][m];
+  for (int m = 0; m < 5; m++) w[m] = sro * s(2, m) + s(4, m);
   interp5<ODR, T, INRANGE, S8>(w, wl[3], wr[3]);
 #pragma unroll
-  for (int m = 0; m < 5; m++) w[m] = sro * s[2][m] - s[4][m];
+  for (int m = 0; m < 5; m++) w[m] = sro * s(2, m) - s(4, m);
   interp5<ODR, T, INRANGE, S8>(w, wl[4], wr[4]);
+  s.again();
 #pragma unroll
-  for (int m = 0; m < 5; m++) w[m] = sro * s[3][m] + s[5][m];
+  for (int m = 0; m < 5; m++) w[m] = sro * s(3, m) + s(5, m);
   interp5<ODR, T, INRANGE, S8>(w, wl[5], wr[5]);
 #pragma unroll
-  for (int m = 0; m < 5; m++) w[m] = sro * s[3][m] - s[5][m];
+  for (int m = 0; m < 5; m++) w[m] = sro * s(3, m) - s(5, m);
   interp5<ODR, T, INRANGE, S8>(w, wl[6], wr[6]);
+  s.again();
 
   // back projection; with S8 the characteristic values are 8 times their
   // own and the exact factor 1/8 sits in the coefficients
@@ -520,17 +526,44 @@ QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int
   const bool fbl = vl[0] <= eps || vl[6] <= eps;
   const bool fbr = vr[0] <= eps || vr[6] <= eps;
   if (fbl) {
-    vl[0] = s[0][2];
-    vl[1] = s[1][2];
-    vl[6] = s[6][2];
+    vl[0] = s(0, 2);
+    vl[1] = s(1, 2);
+    vl[6] = s(6, 2);
   }
   if (fbr) {
-    vr[0] = s[0][2];
-    vr[1] = s[1][2];
-    vr[6] = s[6][2];
+    vr[0] = s(0, 2);
+    vr[1] = s(1, 2);
+    vr[6] = s(6, 2);
   }
   if (fbc) *fbc = (fbl ? 1 : 0) | (fbr ? 2 : 0);
 }
+
+// the stencil as an array s[k][m] in registers
+template <typename T>
+struct RegStencil {
+  const T (&a)[7][5];
+  QAS_HD T operator()(int k, int m) const { return a[k][m]; }
+  QAS_HD void again() const {}
+};
+template <int ODR, typename T, int MODE = 0, bool INRANGE = true, bool WAVEB = std::is_same<T, double>::value>
+QAS_HD void lrstate(const T (&s)[7][5], T bn, T gam, T (&vl)[7], T (&vr)[7], int* fbc = nullptr)
+{
+  lrstate_of<ODR, T, MODE, INRANGE, WAVEB>(RegStencil<T>{s}, bn, gam, vl, vr, fbc);
+}
+
+// the stencil in LDS: field k of the lane's cell at c[k * K], its neighbours
+// along the line M apart
+template <typename T, typename E, int K, int M>
+struct LdsStencil {
+  const E* c;
+  QAS_HD T operator()(int k, int m) const { return (T)c[k * K + (m - 2) * M]; }
+  QAS_HD void again() const
+  {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" ::: "memory");
+#endif
+  }
+};
 
 // face states of the B-flux b_t v_n - b_n v_t (mhd_func.c:163-188); the
 // caller passes the 5-point products bt*vn, the vt stencil and the two

@@ -36,7 +36,7 @@ xsweep2d_fn pick_grav_ysweep(int rmn, int odr)
 xsweep2d_fn pick_grav_xsweep(int rmn, int odr)
 {
 #define QAS_S(R, O) \
-  if (rmn == R && odr == O) return k_sweep2d<0, R, O, double, false, true>;
+  if (rmn == R && odr == O) return k_sweep2d<R, O, double, false, true>;
   QAS_S(0, 1) QAS_S(0, 2) QAS_S(0, 3) QAS_S(0, 4)
   QAS_S(1, 1) QAS_S(1, 2) QAS_S(1, 3) QAS_S(1, 4)
   QAS_S(2, 1) QAS_S(2, 2) QAS_S(2, 3) QAS_S(2, 4)

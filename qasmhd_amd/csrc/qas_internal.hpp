@@ -11,8 +11,9 @@
 namespace qas {
 
 constexpr int NG = 4;       // ghost layers (mhd2d_class.hpp:10)
-constexpr int SEG = 60;     // faces owned by one wavefront segment (64 lanes - 4 halo)
 constexpr int WAVE = 64;
+constexpr int HALO = 4;     // lanes of a run of cells that only feed their neighbours (2 on each side)
+constexpr int SEG = WAVE - HALO;  // cells owned by one wavefront of a transverse or 1D sweep
 constexpr int CFL_MAX_BLOCKS = 1024;
 // accumulator slots: 2D uses 6 (dt/dy Dy of ro mx my mz bz en); 3D uses
 // 5 + 5 (dt/dy Dy and dt/dz Dz of ro mx my mz en)
@@ -70,6 +71,95 @@ __device__ __forceinline__ int xcd_remap(int b, int nb)
   const int x = b % 8, slot = b / 8;
   const int q = nb / 8, r = nb % 8;
   return (x < r) ? x * (q + 1) + slot : r * (q + 1) + (x - r) * q + slot;
+}
+
+// Tiles of a transverse (y, z) sweep: runs of SEG cells down a column group
+// (4 columns).  Either every column group is cut by itself (bundle 0), or the
+// column groups of a bundle are laid end to end, n cells each, and cut into
+// runs whatever column they fall in, so that only a bundle's last run is
+// partly empty.  Cutting by column leaves 4 % of the lanes idle at n = 520,
+// 14 % at 264 and 32 % at 136; but with runs across columns those of
+// neighbouring columns start at different rows, the cells that share a cache
+// line are less close in time, and a run that ends one column and begins the
+// next takes the general index map.  Measured: FP32 y sweep at 2048^2 267 us by
+// column, 291 in bundles of 8, 332 in one bundle; FP64 at 1024^2 98 and 97;
+// 24 domains of 128^2 to 512^2 233 and 219.  So bundles are taken where they
+// save more than 8 % of the tiles of a launch that fills the chip (a single
+// domain of 256^2, one round of workgroups, 17.2 us by column, 17.5 in bundles).
+__host__ __device__ __forceinline__ int line_runs(int ncol, int n) { return (ncol * n + SEG - 1) / SEG; }
+__host__ __device__ __forceinline__ int line_cuts(int n) { return (n - 5 + SEG - 1) / SEG; }  // runs of one column
+__host__ __device__ __forceinline__ int line_tiles(int ncol, int n, int bundle)
+{
+  if (bundle == 0) return ncol * line_cuts(n);
+  const int nb = ncol / bundle;
+  return nb * line_runs(bundle, n) + line_runs(ncol - nb * bundle, n);
+}
+// the bundle for planes of ncol column groups of n cells, `planes` of them in
+// the launch (a batch counts as many): 8 column groups are the 32 columns of a
+// 128-byte line of floats; more where n is small, for few bundles' ends
+inline int line_bundle(int ncol, int n, long long planes)
+{
+  const int b = 8 * ((511 + n) / n);
+  const long long cut = line_tiles(ncol, n, 0), run = line_tiles(ncol, n, b);
+  return (cut * 100 > run * 108 && run * planes >= 768) ? b : 0;
+}
+
+// Tile t in launch order: the column group and row of its first cell, the
+// column groups [c0, c1) it may reach into and the cells it may own (left).
+// By column, tiles start at row 3, the first with a face, the first tile's
+// own cells reach back to row 0 (first) and the last one's on to row n - 1.
+// In a bundle a tile belongs to the column its first cell is in; every column
+// has n / SEG tiles and some have one more (the last ones in launch order).
+// The k-th tiles of all columns (of a bundle's columns) are consecutive.
+struct LineTile {
+  int col, row, c0, c1;
+  int lo, hi;  // own cells: places [lo, hi) after the first
+};
+__host__ __device__ __forceinline__ LineTile line_tile(int t, int ncol, int n, int bundle)
+{
+  LineTile tl;
+  if (bundle == 0) {
+    const int k = t / ncol;
+    tl.col = t - k * ncol;
+    tl.row = 3 + SEG * k;
+    tl.c0 = tl.col;
+    tl.c1 = tl.col + 1;
+    tl.lo = k == 0 ? -3 : 0;
+    tl.hi = k == line_cuts(n) - 1 ? n - tl.row : SEG;
+    return tl;
+  }
+  const int runs = line_runs(bundle, n);
+  const int b = t / runs;
+  t -= b * runs;
+  tl.c0 = b * bundle;
+  tl.c1 = tl.c0 + bundle < ncol ? tl.c0 + bundle : ncol;
+  const int nc = tl.c1 - tl.c0;
+  const int m = n / SEG, rho = n - m * SEG;
+  int col, k;
+  if (t < m * nc) {
+    k = t / nc;
+    col = t - k * nc;
+  } else {
+    col = (SEG * (t - m * nc)) / rho;
+    k = m;
+  }
+  const int first = (col * n + SEG - 1) / SEG + k;  // its place among the bundle's runs
+  tl.col = tl.c0 + col;
+  tl.row = SEG * first - col * n;
+  tl.lo = 0;
+  tl.hi = nc * n - SEG * first < SEG ? nc * n - SEG * first : SEG;
+  return tl;
+}
+// cell d places after the tile's first (d may be negative); before the
+// first or past the last cell it may reach: that cell
+__host__ __device__ __forceinline__ void line_cell(const LineTile& tl, int n, int d, int& col, int& row)
+{
+  col = tl.col;
+  row = tl.row + d;
+  while (row < 0) { row += n; col--; }
+  while (row >= n) { row -= n; col++; }
+  if (col < tl.c0) { col = tl.c0; row = 0; }
+  if (col >= tl.c1) { col = tl.c1 - 1; row = n - 1; }
 }
 
 // The face parts of the B fluxes (emf) and the stored transverse

@@ -14,10 +14,8 @@
 //   emf2d    CUCT corner EMF from both sweeps' face parts   (:91-103, 201-232, 308-339)
 //   ct2d     staggered bx, by update                        (:359-380)
 //            and the bound() of the stage output             (:384-385)
-// A sweep assigns one 64-lane wavefront to 64 consecutive cells of a line;
-// lane l reconstructs cell f0-2+l, neighbour states and fluxes move between
-// lanes by cross-lane shuffles, and the wavefront owns the 60 faces/cells
-// [f0, f0+60).  Everything runs in FP64 with the reference's operation
+// A lane of a sweep reconstructs one cell; neighbour states and fluxes move
+// between lanes (qas_sweep2d.hpp).  Everything runs in FP64 with the reference's operation
 // order (the library is built with -ffp-contract=off).
 #include "qas_device.hpp"
 #include "qas_internal.hpp"
@@ -68,8 +66,6 @@ hipError_t launch_stage2d(qas_ctx* c, const StagePtrs& p, bool faces_only)
   hipStream_t st = c->stream;
   const bool f32 = c->s.precision == 1;
   // 1) y sweep (with the primitives), 2) x sweep
-  const int nsx = (g.nx - 5 + SEG - 1) / SEG;
-  const int nsy = (g.ny - 5 + SEG - 1) / SEG;
   const int prec = c->s.precision;
   xsweep2d_fn fx = prec == 1 ? pick_xsweep2d_f32(c->s.rmn, odr, false)
                              : (prec == 2 ? pick_xsweep2d_fma(c->s.rmn, odr, false) : pick_xsweep2d(c->s.rmn, odr, false));
@@ -84,15 +80,16 @@ hipError_t launch_stage2d(qas_ctx* c, const StagePtrs& p, bool faces_only)
     ps.in[7] = p.enrt;
   }
   if (!fx || !fy) return hipErrorInvalidValue;
-  // y sweep first (one 256-thread workgroup per (4-column group, segment)):
-  // it stores the primitives and leaves dt/dy * Dy in the accumulators; the
-  // x sweep applies the stage sum
-  QAS_LAUNCH(c, QAS_K_SWEEP_Y, fy, (unsigned)(((g.nx + YC - 1) / YC) * nsy), 256, 0, st, p, g, c->bc, gam, nsy,
-             (const BatchInst*)nullptr, (const int*)nullptr, 0, 0);
-  // x sweep: one wavefront per (line, segment), c->xwpb per workgroup
+  // y sweep first (one 256-thread workgroup per run of 60 cells of a
+  // 4-column group): it stores the primitives and leaves dt/dy * Dy in the
+  // accumulators; the x sweep (c->xwpb wavefronts per workgroup) applies the
+  // stage sum
   const unsigned xb = (unsigned)(WAVE * c->xwpb);
-  QAS_LAUNCH(c, QAS_K_SWEEP_X, fx, nblk((long long)nsx * g.ny * WAVE, (int)xb), xb, 0, st, ps, g, c->bc, gam, nsx,
+  const int yb = ysweep2d_bundle(g, false);
+  QAS_LAUNCH(c, QAS_K_SWEEP_Y, fy, (unsigned)ysweep2d_blocks(g, yb), 256, 0, st, p, g, c->bc, gam, yb,
              (const BatchInst*)nullptr, (const int*)nullptr, 0, 0);
+  QAS_LAUNCH(c, QAS_K_SWEEP_X, fx, (unsigned)xsweep2d_blocks(g, c->xwpb), xb, xsweep2d_lds(c->xwpb, f32), st, ps, g,
+             c->bc, gam, 0, (const BatchInst*)nullptr, (const int*)nullptr, 0, 0);
   if (faces_only) return hipGetLastError();
   // 3) corner EMF, 4) CT with the ghost fill of the stage output
   const bool col = (long long)(g.nx - 5) * (g.ny - 5) >= EMF_COL_MIN;
@@ -121,6 +118,7 @@ hipError_t launch_stage2d(qas_ctx* c, const StagePtrs& p, bool faces_only)
   return hipGetLastError();
 }
 
+unsigned xsweep2d_lds(int wpb, bool f32) { return f32 ? x_lds_bytes<float>(WAVE * wpb) : x_lds_bytes<double>(WAVE * wpb); }
 xsweep2d_fn pick_ysweep2d(int rmn, int odr, bool batch) { return pick_ysweep2d_t<double>(rmn, odr, batch); }
 xsweep2d_fn pick_xsweep2d(int rmn, int odr, bool batch) { return pick_xsweep2d_t<double>(rmn, odr, batch); }
 

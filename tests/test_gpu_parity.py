@@ -121,6 +121,33 @@ def test_2d_column_emf_vs_oracle(qas, oracle, rmn, odr, walls):
     assert np.array_equal(out, ref)
 
 
+@pytest.mark.parametrize("nx,ny,rmn,walls", [(1400, 128, 1, False), (1401, 130, 3, True), (2601, 59, 2, True),
+                                             (5000, 16, 0, False)])
+def test_2d_runs_across_columns_and_rows_vs_oracle(qas, oracle, nx, ny, rmn, walls):
+    """Shapes whose y sweep cuts its runs across column groups (short columns,
+    enough tiles to fill the chip), the last bundle and the last column group
+    partly empty, and runs of the x sweep across rows: bit-identical in each
+    x-sweep workgroup size."""
+    from qasmhd_amd import problems
+    p = problems.turbulence2d(n=nx, ny=ny, seed=3, vrms=0.8)
+    dn = np.zeros((3, 8), dtype=int)
+    if walls:
+        dn[0] = [2] * 8
+        dn[1] = [1, 1, -1, 1, 1, -1, 1, 1]
+    _say("2d runs across columns and rows", nx, ny, rmn, walls)
+    cfg = oracle.make_cfg(p.state.shape[1:], p.dx, p.dy, gam=p.gam, rmn=rmn, dn=dn)
+    ref = p.state.copy()
+    h_ref, dt_ref = oracle.run(cfg, ref, 2, 1)
+    assert np.isfinite(ref).all()
+    for xwpb in (1, 2, 4):
+        with qas.Solver(p.state.shape[1:], p.dx, p.dy, gam=p.gam, rmn=rmn, dn=dn) as s:
+            s.set_shape(xwpb, 256)
+            s.upload(p.state)
+            hist, dt_now = s.run(2, flg=1)
+            assert np.array_equal(hist, h_ref) and dt_now == dt_ref
+            assert np.array_equal(s.download(), ref), xwpb
+
+
 def test_step_and_bound_entry_points(qas, oracle):
     """qas_bound / qas_step / qas_cfl_dt individually == bound / ideal / setdt."""
     from qasmhd_amd import problems
