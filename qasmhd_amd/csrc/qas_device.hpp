@@ -104,9 +104,18 @@ QAS_HD T div_3p2(T x)
 // the same x (quot with inv_raw(x)) 4 against 11, root 13 against 18; the
 // HLLD flux forms 8 reciprocals, 4 quotients and 5 roots, which take 28 % of
 // its instructions as operators.
+//
+// FP32 (the mixed path, built with the fast FP32 division and root): the
+// estimates v_rcp_f32 and v_sqrt_f32 themselves (1 ulp), which that division
+// and root wrap in exponent arithmetic for operands below 2^-96 or above
+// 2^126; the same bits between.  One instruction each against 4 to 6: 230 of
+// 1830 per wavefront of the MLAU y sweep.
 template <typename T>
 QAS_HD T inv_raw(T x)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_rcpf(x);
+#endif
   if constexpr (std::is_same<T, double>::value) return rcp_inrange(x);
   else return T(1.0) / x;
 }
@@ -115,6 +124,7 @@ template <typename T>
 QAS_HD T inv(T x)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_rcpf(x);
   if constexpr (std::is_same<T, double>::value) return __builtin_amdgcn_div_fixup(rcp_inrange(x), x, 1.0);
 #endif
   return T(1.0) / x;
@@ -125,6 +135,7 @@ template <typename T>
 QAS_HD T quot(T a, T x, T rx)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, float>::value) return a * rx;
   if constexpr (std::is_same<T, double>::value) {
     const double q = a * rx;
     return __builtin_amdgcn_div_fixup(fma(fma(-x, q, a), rx, q), x, a);
@@ -138,14 +149,14 @@ QAS_HD T quot(T a, T x, T rx)
 template <typename T>
 QAS_HD T ratio(T a, T x)
 {
-  if constexpr (std::is_same<T, double>::value) return quot(a, x, inv_raw(x));
+  if constexpr (std::is_floating_point<T>::value) return quot(a, x, inv_raw(x));
   else return a / x;
 }
 
 template <typename T>
 QAS_HD T half_inv(T x)
 {
-  if constexpr (std::is_same<T, double>::value) return T(0.5) * inv(x);
+  if constexpr (std::is_floating_point<T>::value) return T(0.5) * inv(x);
   else return T(0.5) / x;
 }
 
@@ -153,6 +164,7 @@ template <typename T>
 QAS_HD T root(T x)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_sqrtf(x);
   if constexpr (std::is_same<T, double>::value) {
     const double r = __builtin_amdgcn_rsq(x);
     double g = x * r, h = 0.5 * r;
@@ -202,7 +214,7 @@ QAS_HD T minmod(T a, T b)
 
 // The weights and face values of WCNS-4 (common_interp.c:102-150) from
 // the three denominators d_k = IS_k^2 + eps; IN_RANGE takes the reciprocals
-// with rcp_inrange (FP64, the caller checked the range), else 1.0 / x.
+// with inv_raw (the caller checked the range), else 1.0 / x.
 // Returns 8 fl and 8 fr: the face values without their factor 1/8, which is
 // exact and which lrstate folds into its coefficients.  Products with powers
 // of two go into the following add (fma2, same rounding), and 6 f = 2 (3 f).
@@ -210,7 +222,7 @@ template <bool IN_RANGE, typename T>
 QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl8, T& fr8)
 {
   auto inv = [](T x) -> T {
-    if constexpr (IN_RANGE) return rcp_inrange(x);
+    if constexpr (IN_RANGE) return inv_raw(x);
     else return T(1.0) / x;
   };
   const T s0 = inv(d0);
@@ -273,16 +285,16 @@ QAS_HD void interp5(const T* f, T& fl, T& fr)
     T s1 = a * a;
     T t = f[3] - T(2.0) * f[2] + f[1];
     t = t * t;
-    s0 = (T(1.0) + t / (s0 + eps));
-    s1 = (T(1.0) + t / (s1 + eps));
+    s0 = (T(1.0) + ratio(t, s0 + eps));
+    s1 = (T(1.0) + ratio(t, s1 + eps));
     T w0 = T(0.25) * s0;
     T w1 = T(0.75) * s1;
-    w0 /= (w0 + w1);
+    w0 = ratio(w0, w0 + w1);
     w1 = T(1.0) - w0;
     fl = T(0.5) * (w0 * (-f[1] + T(3.0) * f[2]) + w1 * (f[2] + f[3]));
     w0 = T(0.75) * s0;
     w1 = T(0.25) * s1;
-    w0 /= (w0 + w1);
+    w0 = ratio(w0, w0 + w1);
     w1 = T(1.0) - w0;
     fr = T(0.5) * (w1 * (-f[3] + T(3.0) * f[2]) + w0 * (f[2] + f[1]));
   } else {  // WCNS4
@@ -319,12 +331,19 @@ QAS_HD void interp5(const T* f, T& fl, T& fr)
         fr = T(0.125) * fr;
       }
     };
-    if constexpr (INRANGE && std::is_same<T, double>::value) {
-      // d >= eps = 1e-40 always; d <= 2^700 keeps every 1/d in
-      // [2^-700, 1e40] and both weight sums in [0.65 * 2^-700, 1e40], so
-      // all five reciprocals are inside rcp_inrange's range (NaN fails
-      // the test and takes the division)
-      if ((d0 <= 0x1p700) & (d1 <= 0x1p700) & (d2 <= 0x1p700)) {
+    if constexpr (INRANGE && std::is_floating_point<T>::value) {
+      // d >= eps always (1e-40, FP32 1e-30); d <= 2^700 (FP32 2^120) keeps
+      // every 1/d and both weight sums, at least 0.65 of the smallest 1/d,
+      // where the plain reciprocal is exact enough (rcp_inrange, v_rcp_f32);
+      // NaN fails the test and takes the division.  (FP64 branches per lane:
+      // with a wavefront-uniform branch the HLLD sweeps took 160 VGPRs against
+      // 144.)
+      constexpr T top = sizeof(T) == 8 ? T(0x1p700) : T(0x1p120);
+      bool in = (d0 <= top) & (d1 <= top) & (d2 <= top);
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (sizeof(T) == 4) in = __all(in) != 0;
+#endif
+      if (in) {
         wcns4_weights<true>(f, d0, d1, d2, fl, fr);
         fin();
         return;

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void k_prim1d(StagePtrs p, Geo g, double gam)
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= g.nd) return;
   const double ro = p.in[0][t];
-  const double iro = 1.0 / ro;
+  const double iro = inv(ro);
   const double vx = p.in[1][t] * iro;
   const double vy = p.in[2][t] * iro;
   const double vz = p.in[3][t] * iro;

@@ -20,7 +20,7 @@ template <typename T>
 struct VelOf {
   const double* m;
   const double* ro;
-  __device__ __forceinline__ T operator[](long long q) const { return (T)(m[q] * (1.0 / ro[q])); }
+  __device__ __forceinline__ T operator[](long long q) const { return (T)(m[q] * inv(ro[q])); }
 };
 
 // shock sensor dv of mhd2d_solve.cpp:105-125 at (i, j) after its bound():
@@ -92,19 +92,20 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH &
   }
   __shared__ T sh[9][YC][YRP];  // ro vy vz vx bz cx pr cy by
   __shared__ T so[8][YC][YRP];  // 6 fluxes, upwind and central B-flux parts
+  __shared__ T sv[RMN >= 2 ? 2 : 1][RMN >= 2 ? YRP : 1];  // vx of the columns left and right of the tile
   const int ncg = (g.nx + YC - 1) / YC;
   const int n = g.ny;
   if (L >= line_tiles(ncg, n, bundle)) return;  // whole workgroup
   const LineTile tl = line_tile(L, ncg, n, bundle);
   const long long sy = g.sy;
+  // a tile of interior cells only skips the ghost-index maps (uniform)
+  const bool inner = (tl.col * YC >= NG) && (tl.col * YC + YC - 1 <= g.nx - NG - 1) && (tl.row - 4 >= NG) &&
+                     (tl.row + YR - 5 <= n - NG - 1);
   {
     // Staging computes the primitives of the tile's cells from the stage
     // input state (prim2d_cell, FP64) and rounds them once to the sweep
     // precision T.  The run's own cells are also stored for the x sweep, so
     // every cell of the domain is written by exactly one workgroup.
-    // a tile of interior cells only skips the ghost-index map (uniform)
-    const bool inner = (tl.col * YC >= NG) && (tl.col * YC + YC - 1 <= g.nx - NG - 1) && (tl.row - 4 >= NG) &&
-                       (tl.row + YR - 5 <= n - NG - 1);
     for (int e = threadIdx.x; e < YC * YR; e += blockDim.x) {
       const int c = e % YC, r = e / YC;
       int cg, row;
@@ -132,6 +133,13 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH &
         G(reinterpret_cast<T*>(p.cx))[a] = cx;
         G(reinterpret_cast<T*>(p.cy))[a] = cy;
         if constexpr (GRAV) p.enrt[a] = q.enrt;
+      }
+    }
+    if constexpr (RMN >= 2) {
+      if (inner && threadIdx.x < 2 * YR) {  // (which other workgroups of this launch store: from the state)
+        const int side = threadIdx.x < YR ? 0 : 1, r = (int)threadIdx.x - side * YR;
+        const VelOf<T> vxs{p.in[1], p.in[0]};
+        sv[side][r] = vxs[sy * (tl.row + r - 4) + tl.col * YC + (side ? YC : -1)];
       }
     }
   }
@@ -179,20 +187,29 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH &
   T dv0 = T(0.0), dv1 = T(0.0);
   // the lane's column and face where global arrays are read (lanes past the
   // domain: some cell of it)
-  int lc = 0, sf = 3;
+  int lc = 0, q = 0, sf = 3;
   if constexpr (RMN >= 2 || GRAV) {
-    int cg, q;
+    int cg;
     line_cell(tl, n, lane - 2, cg, q);
     sf = q < 3 ? 3 : (q > n - 3 ? n - 3 : q);
     lc = cg * YC + w > g.nx - 1 ? g.nx - 1 : cg * YC + w;
   }
   if constexpr (RMN >= 2) {
-    // the transverse sensor needs vx of the neighbouring columns, which
-    // other workgroups of this launch store: taken from the state instead,
-    // with the primitive's own expression and rounding
     dv0 = sh[1][w][rb] - sh[1][w][rb - 1];
-    const VelOf<T> vxs{p.in[1], p.in[0]};
-    dv1 = (T)tmin(dv_at<0>(vxs, lc, sf - 1, g, bc), dv_at<0>(vxs, lc, sf, g, bc));
+    // the transverse sensor of this lane's cell; the other one of its face is
+    // the lane before's.  An interior tile has vx of the neighbouring columns
+    // in LDS; elsewhere it comes from the state through the index maps, with
+    // the primitive's own expression and rounding
+    T dvc;
+    if (inner) {
+      const T v = sh[3][w][rb];
+      const T vm = w > 0 ? sh[3][w > 0 ? w - 1 : 0][rb] : sv[0][rb], vp = w < YC - 1 ? sh[3][w < YC - 1 ? w + 1 : 0][rb] : sv[1][rb];
+      dvc = tmin(vp - v, v - vm);
+    } else {
+      const VelOf<T> vxs{p.in[1], p.in[0]};
+      dvc = (T)dv_at<0>(vxs, lc, q, g, bc);
+    }
+    dv1 = tmin((T)__shfl_up(dvc, 1, WAVE), dvc);
   }
   riemann<RMN>(Lf, Rf, bnf, (T)gam, dv0, dv1, F);
   const T fc = T(0.5) * (qlf + qr);
@@ -249,7 +266,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH &
 // registers: from LDS it gained nothing (142 VGPRs as before, 83.3 us against
 // 82.2 at 1024^2; held to 4 waves per SIMD it spilled, 105 us).
 // LDS per lane: the cell's 7 values (then its 6 fluxes) and, apart from them,
-// 8 face values; odd strides, so that 64 lanes fall on different banks.
+// 8 face values and the sensor; odd strides, so that 64 lanes fall on different banks.
 constexpr int XS = 7, XL = 9;
 template <typename T>
 constexpr unsigned x_lds_bytes(int nb) { return (unsigned)((XS * (nb + HALO) + XL * nb) * sizeof(T)); }
@@ -371,6 +388,18 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 4 : 1) : 3) void 
 #pragma unroll
   for (int k = 0; k < 7; k++) xl[k] = vl[k];
   xl[7] = ql;
+  // the transverse sensor of this lane's cell, handed over too
+  T dvc = T(0.0);
+  if constexpr (RMN >= 2) {
+    const auto vy = G(pv.vy);
+    if (__all((q >= NG) & (q <= n - NG - 1) & (line >= NG) & (line <= g.ny - NG - 1))) {
+      const T v = s(2, 2);
+      dvc = tmin(vy[cell.a + g.sy] - v, v - vy[cell.a - g.sy]);
+    } else {
+      dvc = (T)dv_at<1>(pv.vy, q, line, g, bc);
+    }
+    xl[8] = dvc;
+  }
   __syncthreads();
   const T* const xb = threadIdx.x > 0 ? xl - XL : xl;
   T L[7], F[7];
@@ -383,7 +412,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 4 : 1) : 3) void 
   T dv0 = T(0.0), dv1 = T(0.0);
   if constexpr (RMN >= 2) {
     dv0 = vnf - vnb;
-    dv1 = (T)tmin(dv_at<1>(pv.vy, qf - 1, line, g, bc), dv_at<1>(pv.vy, qf, line, g, bc));
+    dv1 = tmin(xb[8], dvc);
   }
   riemann<RMN>(L, vr, bnf, (T)gam, dv0, dv1, F);
   const T fc = T(0.5) * (qlf + qr);

@@ -56,6 +56,36 @@ def test_mixed_l1_error(case):
     assert e_ro < tol and e_pr < tol
 
 
+@pytest.mark.parametrize("rmn", [1, 3])
+def test_mixed_across_units(rmn):
+    """The same flow in units whose speeds are 2^k times larger: FP32 scales
+    exactly but for the range of its reciprocals, and the WCNS smoothness
+    denominators (of pressures squared, to the fourth power) run from far
+    below to above 2^120, where the weights take the division instead of the
+    estimate.  The error against the FP64 path keeps the bound it has in the
+    first units (test_mixed_l1_error)."""
+    from qasmhd_amd import capi, problems
+    p = problems.turbulence2d(n=64, seed=3)
+    with capi.solver_for(p, rmn=rmn) as s:
+        s.upload(p.state)
+        dt = s.cfl_dt()
+    for k in (0, 8, 12, 13, 14):  # (at 2^15 the denominators overflow FP32)
+        q = p.copy()
+        f = 2.0 ** k
+        q.state[1:7] *= f
+        q.state[7] *= f * f
+        out = []
+        for precision in (0, 1):
+            with capi.solver_for(q, rmn=rmn, precision=precision) as s:
+                s.upload(q.state)
+                s.run(20, flg=0, dt=dt / f, history=False)
+                out.append(s.download())
+        I = (slice(4, -4), slice(4, -4))
+        e = l1rel(out[1][0][I], out[0][0][I])
+        _say("mixed vs fp64, speeds x 2^%d, rmn %d: L1(rho) %.3e" % (k, rmn, e))
+        assert np.isfinite(out[1]).all() and e < 1e-4
+
+
 def test_mixed_l1_error_vs_oracle(oracle):
     """The mixed path's L1 error measured against the oracle itself (the
     CPU restatement of the reference) rather than through the FP64 HIP
