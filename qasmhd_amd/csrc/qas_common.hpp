@@ -14,45 +14,48 @@ struct BoundArgs {
   double gfac = 0.0;            // (2 - gam) / (gam - 1)
 };
 
-// fv(m): the array of variable m (a kernel argument's entry, or a pointer
-// read from an instance table in device memory: a local copy of the
-// pointer array indexed by m would sit in scratch memory); skip(m, s):
-// the ghosts of variable m whose source is cell s are written elsewhere
-template <typename FV, typename SKIP>
-__host__ __device__ __forceinline__ void bound_at_f(const FV& fv, const SKIP& skip, int nvar, const double* phi,
-                                           double gfac, const Geo& g, const BcFlags& bc, long long nghost, int ox,
-                                           int oy, int oz, long long t)
+// ghost cell r of an array (nx, ny, nz with ox, oy, oz ghost layers): z slabs,
+// then y slabs of the inner z range, then x slabs of the inner (y, z) range;
+// 32-bit arithmetic (an array holds fewer than 2^31 cells)
+__host__ __device__ __forceinline__ void ghost_cell(const Geo& g, int ox, int oy, int oz, unsigned r, int& i, int& j,
+                                                    int& k)
 {
-  if (t >= nghost * nvar) return;
-  const int m = (int)(t / nghost);
-  long long r = t - (long long)m * nghost;
-  // decode ghost cell r: z slabs, then y slabs of the inner z range, then
-  // x slabs of the inner (y, z) range
-  const long long nx = g.nx, ny = g.ny, nz = g.nz;
-  const long long zs = 2LL * oz * ny * nx;
-  const long long ys = 2LL * oy * nx * (nz - 2 * oz);
-  int i, j, k;
+  const unsigned nx = (unsigned)g.nx, ny = (unsigned)g.ny, nz = (unsigned)g.nz;
+  const unsigned zs = 2u * oz * ny * nx;
+  const unsigned ys = 2u * oy * nx * (nz - 2 * oz);
   if (r < zs) {
-    const long long plane = r / (ny * nx);
-    const long long rem = r - plane * ny * nx;
-    k = (int)(plane < oz ? plane : nz - 2 * oz + plane);
-    j = (int)(rem / nx);
-    i = (int)(rem % nx);
+    const unsigned line = r / nx, plane = line / ny;
+    i = (int)(r - line * nx);
+    j = (int)(line - plane * ny);
+    k = (int)plane < oz ? (int)plane : (int)nz - 2 * oz + (int)plane;
   } else if (r < zs + ys) {
     r -= zs;
-    const long long row = r / nx;  // 0 .. 2*oy*(nz-2oz)-1
-    i = (int)(r % nx);
-    k = oz + (int)(row / (2 * oy));
-    const int jj = (int)(row % (2 * oy));
+    const unsigned row = r / nx, pl = row / (2u * oy);  // row 0 .. 2*oy*(nz-2oz)-1
+    i = (int)(r - row * nx);
+    k = oz + (int)pl;
+    const int jj = (int)(row - pl * 2u * oy);
     j = jj < oy ? jj : (int)ny - 2 * oy + jj;
   } else {
     r -= zs + ys;
-    const long long col = r % (2 * ox);
-    const long long line = r / (2 * ox);
-    i = (int)(col < ox ? col : nx - 2 * ox + col);
-    j = oy + (int)(line % (ny - 2 * oy));
-    k = oz + (int)(line / (ny - 2 * oy));
+    const unsigned line = r / (2u * ox), pl = line / (ny - 2 * oy);
+    const int col = (int)(r - line * 2u * ox);
+    i = col < ox ? col : (int)nx - 2 * ox + col;
+    j = oy + (int)(line - pl * (ny - 2 * oy));
+    k = oz + (int)pl;
   }
+}
+
+// bound() of variable m at ghost cell (i, j, k).  fv(m): the array of variable
+// m (a kernel argument's entry, or a pointer read from an instance table in
+// device memory: a local copy of the pointer array indexed by m would sit in
+// scratch memory); skip(m, s): the ghosts of variable m whose source is cell s
+// are written elsewhere
+template <typename FV, typename SKIP>
+__host__ __device__ __forceinline__ void bound_cell(const FV& fv, const SKIP& skip, int m, int nvar, const double* phi,
+                                                    double gfac, const Geo& g, const BcFlags& bc, int ox, int oy, int oz,
+                                                    int i, int j, int k)
+{
+  const long long nx = g.nx, ny = g.ny;
   if (phi && m == 7 && nvar == 8 && oz == 0 && (j < oy || j >= ny - oy)) {
     // with gravity along y the energy's y ghosts (x ghosts included) are
     // the hydrostatic extrapolation from the first / last interior row, as
@@ -81,17 +84,24 @@ __host__ __device__ __forceinline__ void bound_at_f(const FV& fv, const SKIP& sk
   fv(m)[(long long)nx * (ny * k + j) + i] = v;
 }
 
+// one variable of one ghost cell per thread
+template <typename FV, typename SKIP>
+__host__ __device__ __forceinline__ void bound_at_f(const FV& fv, const SKIP& skip, int nvar, const double* phi,
+                                           double gfac, const Geo& g, const BcFlags& bc, long long nghost, int ox,
+                                           int oy, int oz, long long t)
+{
+  if (t >= nghost * nvar) return;
+  const int m = (int)(t / nghost);
+  int i, j, k;
+  ghost_cell(g, ox, oy, oz, (unsigned)(t - (long long)m * nghost), i, j, k);
+  bound_cell(fv, skip, m, nvar, phi, gfac, g, bc, ox, oy, oz, i, j, k);
+}
+
 template <typename FV>
 __host__ __device__ __forceinline__ void bound_at_f(const FV& fv, int nvar, const double* phi, double gfac, const Geo& g,
                                            const BcFlags& bc, long long nghost, int ox, int oy, int oz, long long t)
 {
   bound_at_f(fv, [](int, long long) { return false; }, nvar, phi, gfac, g, bc, nghost, ox, oy, oz, t);
-}
-
-__device__ __forceinline__ void bound_at(const BoundArgs& a, const Geo& g, const BcFlags& bc, long long nghost,
-                                         int ox, int oy, int oz, long long t)
-{
-  bound_at_f([&](int m) { return a.f[m]; }, a.nvar, a.phi, a.gfac, g, bc, nghost, ox, oy, oz, t);
 }
 
 struct CflArgs {

@@ -1104,14 +1104,14 @@ QAS_HD T cuct_weight(T ro0, T ro1, T ro2, T ro3, T va0, T va1, T va2, T va3, T v
 {
   const T eps = T(1e-12);
   T roc = T(0.25) * (ro0 + ro1 + ro2 + ro3);
-  roc = T(1.0) / dsqrt(roc);
+  roc = inv(root(roc));
   T vac = T(0.25) * (va0 + va1 + va2 + va3);
   T vbc = T(0.25) * (vb0 + vb1 + vb2 + vb3);
   const T bac = T(0.5) * (ba1 + ba3);
   const T bbc = T(0.5) * (bb2 + bb3);
   vac = dabs(vac) + dabs(bac * roc);
   vbc = dabs(vbc) + dabs(bbc * roc);
-  return (vac + T(0.5) * eps) / (vac + vbc + eps);
+  return ratio(vac + T(0.5) * eps, vac + vbc + eps);
 }
 
 // rk_updt (common/common_func.h:28-32)

@@ -148,6 +148,38 @@ def test_2d_runs_across_columns_and_rows_vs_oracle(qas, oracle, nx, ny, rmn, wal
             assert np.array_equal(s.download(), ref), xwpb
 
 
+@pytest.mark.parametrize("nx,ny,nz,rmn,odr,walls", [(41, 40, 90, 1, 4, False), (41, 40, 90, 3, 4, True),
+                                                    (300, 9, 17, 2, 2, True), (17, 130, 8, 0, 3, False)])
+def test_3d_runs_chunks_and_ghosts_vs_oracle(qas, oracle, nx, ny, nz, rmn, odr, walls):
+    """3D shapes whose y and z sweeps cut their runs across column groups
+    (short columns, many planes) or by column, with partly empty last groups;
+    edge and face marches with a partly empty last chunk; planes that do not
+    divide into workgroups; every boundary kind: bit-identical."""
+    rng = np.random.default_rng(nx + ny)
+    shape = (nz + 8, ny + 8, nx + 8)
+    z, y, x = np.meshgrid(*[2 * np.pi * (np.arange(n) - 4) / (n - 8) for n in shape], indexing="ij")
+    f = [sum(rng.uniform(0.2, 0.5) * np.cos(a * x + b * y + c * z + rng.uniform(0, 6)) for a, b, c in
+             ((1, 0, 1), (0, 1, 1), (1, 1, 0))) for _ in range(8)]
+    st = np.stack([1.5 + 0.3 * f[0], f[1], f[2], f[3], f[4], f[5], f[6], 8.0 + f[7]])
+    dn = np.zeros((3, 8), dtype=int)
+    if walls:
+        dn[0] = [2] * 8
+        dn[1] = [1, 1, -1, 1, 1, -1, 1, 1]
+        dn[2] = [-2 if m == 3 else 2 for m in range(8)]
+    _say("3d runs, chunks and ghosts", nx, ny, nz, rmn, odr, walls)
+    d = 2 * np.pi / max(nx, ny, nz)
+    cfg = oracle.make_cfg(shape, d, d, d, rmn=rmn, odr=odr, dn=dn)
+    ref = st.copy()
+    h_ref, dt_ref = oracle.run(cfg, ref, 2, 1)
+    assert np.isfinite(ref).all()
+    with qas.Solver(shape, d, d, d, rmn=rmn, odr=odr, dn=dn) as s:
+        s.upload(st)
+        hist, dt_now = s.run(2, flg=1)
+        out = s.download()
+    assert np.array_equal(hist, h_ref) and dt_now == dt_ref
+    assert np.array_equal(out, ref)
+
+
 def test_step_and_bound_entry_points(qas, oracle):
     """qas_bound / qas_step / qas_cfl_dt individually == bound / ideal / setdt."""
     from qasmhd_amd import problems
