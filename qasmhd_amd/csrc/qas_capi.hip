@@ -337,11 +337,12 @@ int qas::ctx_step(qas_ctx* c)
   for (int rk = 0; rk < R; rk++) {
     const StagePtrs p = stage_ptrs(c, rk, seq_in[rk], seq_out[rk], A);
     hipError_t e;
+    // (1D and 2D stages fill the ghosts of their output themselves)
     if (c->g.ndim == 1) e = launch_stage1d(c, p);
-    else if (c->g.ndim == 2) e = launch_stage2d(c, p);  // ghost fill inside the CT launch
+    else if (c->g.ndim == 2) e = launch_stage2d(c, p);
     else e = launch_stage3d(c, p);
     if (e != hipSuccess) return hipfail(c, e, "stage launch");
-    if (c->g.ndim != 2) {
+    if (c->g.ndim == 3) {
       e = launch_bound(c, c->U[seq_out[rk]], 8);
       if (e != hipSuccess) return hipfail(c, e, "bound launch");
     }

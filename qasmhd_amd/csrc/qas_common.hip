@@ -81,6 +81,22 @@ hipError_t launch_bound(qas_ctx* c, double* const f[8], int nvar)
 // ------------------------------------------------------------------ CFL
 __global__ __launch_bounds__(256) void k_cfl(CflArgs a, Geo g) { cfl_block(a, g, (int)blockIdx.x, (int)gridDim.x); }
 
+// A small domain's whole reduction in one workgroup of 1024 threads (up to
+// CFL_ONE cells, 4 per thread): the second launch cost 3.8 us, as much as
+// the first (64^2 and 1D: 4.2 + 3.8 us, one workgroup 3.9).
+constexpr long long CFL_ONE = 4096;
+__global__ __launch_bounds__(1024) void k_cfl_one(CflArgs a, Geo g, double* dt, double cfl_dr)
+{
+  __shared__ double wm[16];
+  double v = wave_max(cfl_thread(a, g, 0, 1));
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; w++) v = (wm[w] > v) ? wm[w] : v;
+    *dt = cfl_dr / v;
+  }
+}
+
 __global__ __launch_bounds__(256) void k_cfl_final(const double* part, int nb, double* dt, double* hist_slot,
                                                    double cfl_dr)
 {
@@ -95,6 +111,18 @@ __global__ void k_record(const double* dt, double* hist, long long* cnt, long lo
   const long long n = *cnt;
   if (n < cap) hist[n] = *dt;
   *cnt = n + 1;
+}
+
+// the smallest cell size of the active axes
+static double cell_size(const Geo& g)
+{
+  double dr = g.dx;
+  if (g.ndim == 2) dr = (g.dx >= g.dy) ? g.dy : g.dx;
+  if (g.ndim == 3) {
+    const double t = (g.dx >= g.dy) ? g.dy : g.dx;
+    dr = (t >= g.dz) ? g.dz : t;
+  }
+  return dr;
 }
 
 hipError_t launch_cfl(qas_ctx* c, const double* const U[8])
@@ -114,6 +142,11 @@ hipError_t launch_cfl(qas_ctx* c, const double* const U[8])
   }
   const int ox = qas::NG, oy = g.ndim >= 2 ? qas::NG : 0, oz = g.ndim >= 3 ? qas::NG : 0;
   const long long n = (long long)(g.nx - 2 * ox) * (g.ny - 2 * oy) * (g.nz - 2 * oz);
+  if (n <= CFL_ONE) {
+    c->cfl_blocks = 0;
+    QAS_LAUNCH(c, QAS_K_CFL, k_cfl_one, 1, 1024, 0, c->stream, a, g, c->d_dt, c->s.cfl * cell_size(g));
+    return hipGetLastError();
+  }
   long long nb = (n + 255) / 256;
   if (nb > CFL_MAX_BLOCKS) nb = CFL_MAX_BLOCKS;
   c->cfl_blocks = (int)nb;
@@ -123,14 +156,8 @@ hipError_t launch_cfl(qas_ctx* c, const double* const U[8])
 
 hipError_t launch_cfl_finalize(qas_ctx* c, double* hist_slot)
 {
-  const Geo& g = c->geo;
-  double dr = g.dx;
-  if (g.ndim == 2) dr = (g.dx >= g.dy) ? g.dy : g.dx;
-  if (g.ndim == 3) {
-    const double t = (g.dx >= g.dy) ? g.dy : g.dx;
-    dr = (t >= g.dz) ? g.dz : t;
-  }
-  const double cfl_dr = c->s.cfl * dr;
+  if (c->cfl_blocks == 0) return hipGetLastError();  // k_cfl_one has set dt
+  const double cfl_dr = c->s.cfl * cell_size(c->geo);
   hipLaunchKernelGGL(k_cfl_final, 1, 256, 0, c->stream, c->d_cflpart, c->cfl_blocks, c->d_dt, hist_slot, cfl_dr);
   return hipGetLastError();
 }

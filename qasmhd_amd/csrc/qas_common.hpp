@@ -136,9 +136,9 @@ __device__ __forceinline__ double block_max(double v)
   return v;
 }
 
-// grid-stride over the interior; each block writes its maximum of
-// |v| + vfast (floor 1.0, the reference's initial vmax) to part[block]
-__device__ __forceinline__ void cfl_block(const CflArgs& a, const Geo& g, int blk, int nblk)
+// grid-stride over the interior: the thread's maximum of |v| + vfast (floor
+// 1.0, the reference's initial vmax)
+__device__ __forceinline__ double cfl_thread(const CflArgs& a, const Geo& g, int blk, int nblk)
 {
   const int ox = qas::NG;
   const int oy = g.ndim >= 2 ? qas::NG : 0;
@@ -186,7 +186,13 @@ __device__ __forceinline__ void cfl_block(const CflArgs& a, const Geo& g, int bl
     else v = sqrt(vx * vx + vy * vy + vz * vz) + vf;
     if (v > vm) vm = v;
   }
-  vm = block_max(vm);
+  return vm;
+}
+
+// each block writes its maximum to part[block]
+__device__ __forceinline__ void cfl_block(const CflArgs& a, const Geo& g, int blk, int nblk)
+{
+  const double vm = block_max(cfl_thread(a, g, blk, nblk));
   if (threadIdx.x == 0) a.part[blk] = vm;
 }
 

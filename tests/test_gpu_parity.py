@@ -180,6 +180,37 @@ def test_3d_runs_chunks_and_ghosts_vs_oracle(qas, oracle, nx, ny, nz, rmn, odr, 
     assert np.array_equal(out, ref)
 
 
+@pytest.mark.parametrize("n", [8, 52, 53, 57, 112, 4097])
+@pytest.mark.parametrize("dn", [0, 1, -1, 2, -2])
+def test_1d_stage_and_ghosts_vs_oracle(qas, oracle, n, dn):
+    """The 1D stage's one launch at the ends of its 60-cell wavefronts, with
+    every boundary kind (bx is staggered along x, so its last face is kept
+    though not evolved), and the CFL reduction in one workgroup or two
+    launches: bit-identical, ghosts included."""
+    rng = np.random.default_rng(n)
+    x = 2 * np.pi * np.arange(n + 8) / n
+    f = [rng.uniform(0.1, 0.3) * np.sin(x + rng.uniform(0, 6)) for _ in range(8)]
+    st = np.stack([1.0 + f[0], f[1], f[2], f[3], 0.7 + f[4], 0.5 + f[5], f[6], 4.0 + f[7]])
+    flags = np.zeros((3, 8), dtype=int)
+    flags[0] = dn
+    flags[0, [0, 7]] = abs(dn)          # density and energy keep their sign
+    flags[0, 4] = 2 if dn == -2 else dn  # (a zero normal field would stop the run)
+    _say("1d stage and ghosts", n, dn)
+    cfg = oracle.make_cfg((n + 8,), 1.0 / n, gam=1.4, dn=flags)
+    ref = st.copy()
+    oracle.bound(cfg, ref)
+    h_ref, dt_ref = oracle.run(cfg, ref, 3, 1)
+    with qas.Solver((n + 8,), 1.0 / n, gam=1.4, dn=flags) as s:
+        s.upload(st)
+        s.bound()
+        hist, dt_now = s.run(3, flg=1)
+        out = s.download()
+    if dn != -2:
+        assert np.isfinite(ref).all()
+    assert np.array_equal(hist, h_ref, equal_nan=True) and np.array_equal(dt_now, dt_ref, equal_nan=True)
+    assert np.array_equal(out, ref, equal_nan=True)
+
+
 def test_step_and_bound_entry_points(qas, oracle):
     """qas_bound / qas_step / qas_cfl_dt individually == bound / ideal / setdt."""
     from qasmhd_amd import problems
