@@ -84,12 +84,8 @@ __device__ __forceinline__ double vel(const StagePtrs& p, int comp, long long c)
 // ------------------------------------------------------------------ EMF
 // FT: element type of the face parts (the sweep precision)
 template <int ODR, typename FT>
-__device__ __forceinline__ void emf2d_at(const StagePtrs& p, const Geo& g, int ctw, long long t)
+__device__ __forceinline__ double emf2d_corner(const StagePtrs& p, const Geo& g, int ctw, int i, int j)
 {
-  const int ni = g.nx - 5, nj = g.ny - 5;   // corners [3, n-3]
-  if (t >= (long long)ni * nj) return;
-  const int i = 3 + (int)(t % ni);
-  const int j = 3 + (int)(t / ni);
   const long long nx = g.nx;
   const long long ss = nx * j + i;
   double ct = 0.5;
@@ -135,7 +131,17 @@ __device__ __forceinline__ void emf2d_at(const StagePtrs& p, const Geo& g, int c
     lin5<ODR>(b, dum, ur1);
     ez += +0.5 * ((ul0 + ur0) + ct * (ul1 + ur1));
   }
-  p.ez[ss] = ez;
+  return ez;
+}
+
+// corners [3, n-3] one per thread
+template <int ODR, typename FT>
+__device__ __forceinline__ void emf2d_at(const StagePtrs& p, const Geo& g, int ctw, long long t)
+{
+  const int ni = g.nx - 5, nj = g.ny - 5;
+  if (t >= (long long)ni * nj) return;
+  const int i = 3 + (int)(t % ni), j = 3 + (int)(t / ni);
+  p.ez[(long long)g.nx * j + i] = emf2d_corner<ODR, FT>(p, g, ctw, i, j);
 }
 
 // CJ corners (i, j0 .. j0 + CJ - 1) of one column per thread, each with
@@ -238,20 +244,29 @@ __device__ __forceinline__ void emf2d_col(const StagePtrs& p, const Geo& g, int 
 // ------------------------------------------------------------------ CT
 // the new bx (comp 0, faces i in [4, nx-4], rows j in [4, ny-5]) or by
 // (comp 1, i in [4, nx-5], j in [4, ny-4]) at face ss
+// ez(di, dj): the corner EMF at (i + di, j + dj)
+template <int ODR, typename EZ>
+__host__ __device__ __forceinline__ double ct2d_face_of(const EZ& ez, const StagePtrs& p, const Geo& g, long long ss,
+                                                        int comp)
+{
+  const double dtv = G(p.dt)[0];
+  if (comp == 0) {
+    const double dtdy = dtv / g.dy;
+    const double du = dfc<ODR>(ez(0, -1), ez(0, 0), ez(0, 1), ez(0, 2));
+    return rk_upd(G(p.in[4])[ss], G(p.u0[4])[ss], -dtdy * du, p.a, p.b);
+  }
+  const double mdtdx = -(dtv / g.dx);  // mhd_updt2d_ctb is called with -dtdx
+  const double du = dfc<ODR>(ez(-1, 0), ez(0, 0), ez(1, 0), ez(2, 0));
+  return rk_upd(G(p.in[5])[ss], G(p.u0[5])[ss], -mdtdx * du, p.a, p.b);
+}
+
+// the same with the corner EMFs in memory
 template <int ODR>
 __host__ __device__ __forceinline__ double ct2d_face(const StagePtrs& p, const Geo& g, long long ss, int comp)
 {
   const long long nx = g.nx;
-  const double dtv = G(p.dt)[0];
   const auto ez = G(p.ez);
-  if (comp == 0) {
-    const double dtdy = dtv / g.dy;
-    const double du = dfc<ODR>(ez[ss - nx], ez[ss], ez[ss + nx], ez[ss + 2 * nx]);
-    return rk_upd(G(p.in[4])[ss], G(p.u0[4])[ss], -dtdy * du, p.a, p.b);
-  }
-  const double mdtdx = -(dtv / g.dx);  // mhd_updt2d_ctb is called with -dtdx
-  const double du = dfc<ODR>(ez[ss - 1], ez[ss], ez[ss + 1], ez[ss + 2]);
-  return rk_upd(G(p.in[5])[ss], G(p.u0[5])[ss], -mdtdx * du, p.a, p.b);
+  return ct2d_face_of<ODR>([&](int di, int dj) -> double { return ez[ss + di + nx * dj]; }, p, g, ss, comp);
 }
 
 // CT alone (the batched stages, whose ghost fill is its own launch)
@@ -332,6 +347,41 @@ __host__ __device__ __forceinline__ void push_ghosts(double* f, int nx, int ny, 
   }
 }
 
+// The CT update of the faces (i, j), i, j in [4, n-4] (bx for j <= ny-5, by for
+// i <= nx-5), except those that bound() overwrites (the periodic image of the
+// last face), and each updated face's ghost images.  ez(di, dj): the corner EMF
+// at (i + di, j + dj)
+template <int ODR, typename EZ>
+__host__ __device__ __forceinline__ void ctb2d_face(const EZ& ez, const StagePtrs& p, const Geo& g, const BcFlags& bc,
+                                                    int i, int j)
+{
+  const int nx = g.nx, ny = g.ny;
+  const long long ss = (long long)nx * j + i;
+  // only faces within 2 NG + 1 of an edge are ghost sources or ghosts
+  bool w4 = j <= ny - 5, w5 = i <= nx - 5;
+  unsigned mx4 = 0, my4 = 0, mx5 = 0, my5 = 0;
+  if (i <= 2 * NG || i >= nx - 2 * NG - 1 || j <= 2 * NG || j >= ny - 2 * NG - 1) {
+    w4 = w4 && !bound_writes(g, bc, 4, i, j);
+    w5 = w5 && !bound_writes(g, bc, 5, i, j);
+    mx4 = ghost_images(i, nx, bc.st[0][4], bc.dn[0][4]);
+    my4 = ghost_images(j, ny, bc.st[1][4], bc.dn[1][4]);
+    mx5 = ghost_images(i, nx, bc.st[0][5], bc.dn[0][5]);
+    my5 = ghost_images(j, ny, bc.st[1][5], bc.dn[1][5]);
+  }
+  const Src fx4 = resolve(0, nx, bc.st[0][4], bc.dn[0][4]), fy4 = resolve(0, ny, bc.st[1][4], bc.dn[1][4]);
+  const Src fx5 = resolve(0, nx, bc.st[0][5], bc.dn[0][5]), fy5 = resolve(0, ny, bc.st[1][5], bc.dn[1][5]);
+  double* o4 = p.out[4];
+  double* o5 = p.out[5];
+  const double v4 = w4 ? ct2d_face_of<ODR>(ez, p, g, ss, 0) : 0.0;
+  const double v5 = w5 ? ct2d_face_of<ODR>(ez, p, g, ss, 1) : 0.0;
+  if (w4) o4[ss] = v4;
+  if (w5) o5[ss] = v5;
+  if ((mx4 | my4 | mx5 | my5) != 0) {
+    if (w4) push_ghosts(o4, nx, ny, i, j, mx4, my4, fx4, fy4, v4);
+    if (w5) push_ghosts(o5, nx, ny, i, j, mx5, my5, fx5, fy5, v5);
+  }
+}
+
 // CT fused with the ghost fill of the stage output (one launch instead of
 // ct2d + bound).  Thread t < nc updates the faces (i, j) with i, j in
 // [4, n-4] (bx for j <= ny-5, by for i <= nx-5), except those that bound()
@@ -344,42 +394,17 @@ template <int ODR>
 __host__ __device__ __forceinline__ void ctb2d_at(const StagePtrs& p, const Geo& g, const BcFlags& bc, const double* phi,
                                          double gfac, long long nghost, long long t, bool ct_part)
 {
+  const long long nx = g.nx;
   if (ct_part) {
-    const int nx = g.nx, ny = g.ny;
-    const int ni = nx - 7, nj = ny - 7;
+    const int ni = g.nx - 7, nj = g.ny - 7;
     if (t >= (long long)ni * nj) return;
     const int i = 4 + (int)(t % ni);
     const int j = 4 + (int)(t / ni);
-    const long long ss = (long long)nx * j + i;
-    // everything read from the arguments before the first store (a batched
-    // launch reads them from its instance table, which the compiler must
-    // otherwise reload after each store)
-    // only faces within 2 NG + 1 of an edge are ghost sources or ghosts
-    bool w4 = j <= ny - 5, w5 = i <= nx - 5;
-    unsigned mx4 = 0, my4 = 0, mx5 = 0, my5 = 0;
-    if (i <= 2 * NG || i >= nx - 2 * NG - 1 || j <= 2 * NG || j >= ny - 2 * NG - 1) {
-      w4 = w4 && !bound_writes(g, bc, 4, i, j);
-      w5 = w5 && !bound_writes(g, bc, 5, i, j);
-      mx4 = ghost_images(i, nx, bc.st[0][4], bc.dn[0][4]);
-      my4 = ghost_images(j, ny, bc.st[1][4], bc.dn[1][4]);
-      mx5 = ghost_images(i, nx, bc.st[0][5], bc.dn[0][5]);
-      my5 = ghost_images(j, ny, bc.st[1][5], bc.dn[1][5]);
-    }
-    const Src fx4 = resolve(0, nx, bc.st[0][4], bc.dn[0][4]), fy4 = resolve(0, ny, bc.st[1][4], bc.dn[1][4]);
-    const Src fx5 = resolve(0, nx, bc.st[0][5], bc.dn[0][5]), fy5 = resolve(0, ny, bc.st[1][5], bc.dn[1][5]);
-    double* o4 = p.out[4];
-    double* o5 = p.out[5];
-    const double v4 = w4 ? ct2d_face<ODR>(p, g, ss, 0) : 0.0;
-    const double v5 = w5 ? ct2d_face<ODR>(p, g, ss, 1) : 0.0;
-    if (w4) o4[ss] = v4;
-    if (w5) o5[ss] = v5;
-    if ((mx4 | my4 | mx5 | my5) != 0) {
-      if (w4) push_ghosts(o4, nx, ny, i, j, mx4, my4, fx4, fy4, v4);
-      if (w5) push_ghosts(o5, nx, ny, i, j, mx5, my5, fx5, fy5, v5);
-    }
+    const long long ss = nx * j + i;
+    const auto ez = G(p.ez);
+    ctb2d_face<ODR>([&](int di, int dj) -> double { return ez[ss + di + nx * dj]; }, p, g, bc, i, j);
     return;
   }
-  const long long nx = g.nx;
   auto pushed = [&](int m, long long s) {
     return (m == 4 || m == 5) && ct_range(g, m, (int)(s % nx), (int)(s / nx));
   };
