@@ -187,7 +187,7 @@ extern "C" int qas_create(qas_ctx** out, const qas_grid* g, const qas_scheme* s)
   if (e != hipSuccess) return fail(c, QAS_E_NOMEM, std::string("hipMalloc of the domain failed: ") + hipGetErrorName(e));
   ctx_layout(c, (char*)c->slab, nullptr);
   QAS_CHECK(c, hipMemsetAsync(c->slab, 0, c->slab_bytes, c->stream));
-  QAS_CHECK(c, hipHostMalloc((void**)&c->h_pinned, 64 * sizeof(double), hipHostMallocDefault));
+  QAS_CHECK(c, hipHostMalloc((void**)&c->h_pinned, PINNED * sizeof(double), hipHostMallocDefault));
   QAS_CHECK(c, hipStreamSynchronize(c->stream));
   return QAS_OK;
 }
@@ -574,10 +574,18 @@ extern "C" int qas_run(qas_ctx* c, int nsteps, int flg, double* dt_inout, double
     int r = loop_step(c, flg, hist, c->nstep % 2 == 0);
     if (r) return r;
   }
+  // dt and, where it fits the pinned buffer, the history in one wait (a copy
+  // into the caller's pageable memory waits by itself)
+  const bool pinned_hist = hist && nsteps > 0 && nsteps < PINNED;
   QAS_CHECK(c, hipMemcpyAsync(c->h_pinned, c->d_dt, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+  if (pinned_hist)
+    QAS_CHECK(c, hipMemcpyAsync(c->h_pinned + 1, c->d_hist, sizeof(double) * (size_t)nsteps, hipMemcpyDeviceToHost,
+                                c->stream));
   QAS_CHECK(c, hipStreamSynchronize(c->stream));
   *dt_inout = c->h_pinned[0];
-  if (hist && nsteps > 0) {
+  if (pinned_hist) {
+    std::memcpy(dt_hist, c->h_pinned + 1, sizeof(double) * (size_t)nsteps);
+  } else if (hist && nsteps > 0) {
     QAS_CHECK(c, hipMemcpyAsync(dt_hist, c->d_hist, sizeof(double) * (size_t)nsteps, hipMemcpyDeviceToHost,
                                 c->stream));
     QAS_CHECK(c, hipStreamSynchronize(c->stream));

@@ -15,6 +15,7 @@ constexpr int WAVE = 64;
 constexpr int HALO = 4;     // lanes of a run of cells that only feed their neighbours (2 on each side)
 constexpr int SEG = WAVE - HALO;  // cells owned by one wavefront of a transverse or 1D sweep
 constexpr int CFL_MAX_BLOCKS = 1024;
+constexpr int PINNED = 256;  // doubles of a context's pinned staging buffer
 // accumulator slots: 2D uses 6 (dt/dy Dy of ro mx my mz bz en); 3D uses
 // 5 + 5 (dt/dy Dy and dt/dz Dz of ro mx my mz en)
 constexpr int NACC = 12;  // blocks of the CFL reduction (grid-stride)

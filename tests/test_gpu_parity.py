@@ -211,6 +211,24 @@ def test_1d_stage_and_ghosts_vs_oracle(qas, oracle, n, dn):
     assert np.array_equal(out, ref, equal_nan=True)
 
 
+@pytest.mark.parametrize("nsteps", [1, 255, 256, 300])
+def test_history_through_pinned_buffer_or_direct(qas, oracle, nsteps):
+    """The dt history comes back with dt in one wait where it fits the pinned
+    buffer (255 steps) and by a copy of its own beyond: every entry."""
+    from qasmhd_amd import problems
+    p = problems.turbulence2d(n=16, seed=5, vrms=0.3)
+    _say("history", nsteps)
+    cfg = oracle.make_cfg(p.state.shape[1:], p.dx, p.dy, gam=p.gam)
+    ref = p.state.copy()
+    h_ref, dt_ref = oracle.run(cfg, ref, nsteps, 1)
+    with qas.solver_for(p) as s:
+        s.upload(p.state)
+        hist, dt_now = s.run(nsteps, flg=1)
+        out = s.download()
+    assert np.array_equal(hist, h_ref) and dt_now == dt_ref
+    assert np.array_equal(out, ref)
+
+
 def test_step_and_bound_entry_points(qas, oracle):
     """qas_bound / qas_step / qas_cfl_dt individually == bound / ideal / setdt."""
     from qasmhd_amd import problems
