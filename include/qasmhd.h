@@ -263,11 +263,11 @@ int qas_adj_keep_stages(qas_ctx *c, int on);
 
 /* ---- instrumentation (no counterpart in the reference) -----------------
  * Kernel identifiers of one stage, for the timing hooks and the work model. */
-#define QAS_K_PRIM 0      /* cell-centred B + primitives (2D: in SWEEP_Y)   */
+#define QAS_K_PRIM 0      /* primitives: no launch of their own any more     */
 #define QAS_K_SWEEP_X 1   /* reconstruction + Riemann + divergence along x  */
 #define QAS_K_SWEEP_Y 2
 #define QAS_K_SWEEP_Z 3
-#define QAS_K_EMF 4       /* CUCT edge EMFs                                 */
+#define QAS_K_EMF 4       /* CUCT edge EMFs (small 2D domains: in CT)       */
 #define QAS_K_CT 5        /* staggered-B update (2D: with the ghost fill of  */
                           /* the stage output)                              */
 #define QAS_K_BOUND 6     /* ghost fill (2D: before the first step only)    */
