@@ -81,10 +81,10 @@ hipError_t launch_bound(qas_ctx* c, double* const f[8], int nvar)
 // ------------------------------------------------------------------ CFL
 __global__ __launch_bounds__(256) void k_cfl(CflArgs a, Geo g) { cfl_block(a, g, (int)blockIdx.x, (int)gridDim.x); }
 
-// A small domain's whole reduction in one workgroup of 1024 threads (up to
-// CFL_ONE cells, 4 per thread): the second launch cost 3.8 us, as much as
-// the first (64^2 and 1D: 4.2 + 3.8 us, one workgroup 3.9).
-constexpr long long CFL_ONE = 4096;
+// A small domain's whole reduction in one workgroup of 1024 threads, one cell
+// each: 3.9 us at 1024 cells against 3.8 + 3.8 for two launches.  With 4 cells
+// per thread (64^2) it took 10.0 us against 4.2 + 3.8.
+constexpr long long CFL_ONE = 1024;
 __global__ __launch_bounds__(1024) void k_cfl_one(CflArgs a, Geo g, double* dt, double cfl_dr)
 {
   __shared__ double wm[16];
