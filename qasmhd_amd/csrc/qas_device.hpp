@@ -280,23 +280,48 @@ QAS_HD void interp5(const T* f, T& fl, T& fr)
   } else if constexpr (ODR == 3) {  // WCNS3
     const T eps = wcns_eps<T>();
     T a = f[1] - f[2];
-    T s0 = a * a;
+    const T s0 = a * a;
     a = f[3] - f[2];
-    T s1 = a * a;
+    const T s1 = a * a;
     T t = f[3] - T(2.0) * f[2] + f[1];
     t = t * t;
-    s0 = (T(1.0) + ratio(t, s0 + eps));
-    s1 = (T(1.0) + ratio(t, s1 + eps));
-    T w0 = T(0.25) * s0;
-    T w1 = T(0.75) * s1;
-    w0 = ratio(w0, w0 + w1);
-    w1 = T(1.0) - w0;
-    fl = T(0.5) * (w0 * (-f[1] + T(3.0) * f[2]) + w1 * (f[2] + f[3]));
-    w0 = T(0.75) * s0;
-    w1 = T(0.25) * s1;
-    w0 = ratio(w0, w0 + w1);
-    w1 = T(1.0) - w0;
-    fr = T(0.5) * (w1 * (-f[3] + T(3.0) * f[2]) + w0 * (f[2] + f[1]));
+    auto face = [&](auto div) {
+      T u0 = T(1.0) + div(t, s0 + eps);
+      T u1 = T(1.0) + div(t, s1 + eps);
+      if constexpr (std::is_same<T, float>::value) {  // (at most one is that large, and its weight is 1)
+        u0 = tmin(u0, T(0x1p125));
+        u1 = tmin(u1, T(0x1p125));
+      }
+      T w0 = T(0.25) * u0;
+      T w1 = T(0.75) * u1;
+      w0 = div(w0, w0 + w1);
+      w1 = T(1.0) - w0;
+      fl = T(0.5) * (w0 * (-f[1] + T(3.0) * f[2]) + w1 * (f[2] + f[3]));
+      w0 = T(0.75) * u0;
+      w1 = T(0.25) * u1;
+      w0 = div(w0, w0 + w1);
+      w1 = T(1.0) - w0;
+      fr = T(0.5) * (w1 * (-f[3] + T(3.0) * f[2]) + w0 * (f[2] + f[1]));
+    };
+    if constexpr (INRANGE && std::is_floating_point<T>::value) {
+      // t <= 4 max(s0, s1), and eps is 2^-133 (FP32 2^-100): s0, s1 <= 2^700
+      // keep the denominators and the weight sums below 2^837, where the
+      // reciprocal has its precision.  In FP32 2^120 keeps the first
+      // denominators in the range of v_rcp_f32, which gives 0 from 2^126 on;
+      // the weight sums may be t / eps (beside a flat pair, s0 = 0: past 2^126
+      // from a difference of 1.07e4 on, past FP32 from 1.84e4 on) and are
+      // held below 2^126.  NaN fails the test.
+      constexpr T top = sizeof(T) == 8 ? T(0x1p700) : T(0x1p120);
+      bool in = (s0 <= top) & (s1 <= top);
+#if defined(__HIP_DEVICE_COMPILE__)
+      if constexpr (sizeof(T) == 4) in = __all(in) != 0;
+#endif
+      if (in) {
+        face([](T x, T y) { return ratio(x, y); });
+        return;
+      }
+    }
+    face([](T x, T y) { return x / y; });
   } else {  // WCNS4
     const T eps = wcns_eps<T>();
     const T c13 = T(13. / 12.);

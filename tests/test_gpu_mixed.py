@@ -86,6 +86,62 @@ def test_mixed_across_units(rmn):
         assert np.isfinite(out[1]).all() and e < 1e-4
 
 
+@pytest.mark.parametrize("jump", [1e3, 1.1e4, 1.4e4, 1.8e4, 3e4])
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+def test_mixed_wcns3_flat_beside_a_jump(rmn, jump):
+    """ODR 3 where the pressure is flat up to a jump: one smoothness measure
+    is zero, the weights' sum is the jump squared over the FP32 eps (1e-30),
+    and from a jump of 1.07e4 on the sum lies above 2^126, past which the FP32
+    reciprocal estimate gives 0; from 1.84e4 on it overflows FP32.
+    The stencil must stay on the flat side, as in FP64: both pressures'
+    differences are a few FP32 roundings (6e-8 each) after three steps."""
+    from qasmhd_amd import capi
+    n = 32
+    st = np.zeros((8, n + 8, n + 8))
+    st[0], st[4], st[5] = 1.0, 30.0, 20.0
+    pr = np.full((n + 8, n + 8), 3e4)
+    pr[:, (n + 8) // 2:] += jump
+    pr[(n + 8) // 2:] += jump
+    st[7] = pr / (5.0 / 3.0 - 1.0) + 0.5 * (900.0 + 400.0)
+    out = []
+    for precision in (0, 1):
+        with capi.Solver(st.shape[1:], 1.0 / n, 1.0 / n, rmn=rmn, odr=3, precision=precision) as s:
+            s.upload(st)
+            s.run(3, flg=0, dt=0.2 / n / 400.0, history=False)
+            out.append(s.download())
+    I = (slice(4, -4), slice(4, -4))
+    e = [l1rel(out[1][m][I], out[0][m][I]) for m in (0, 7)]
+    _say("mixed odr 3, flat beside a jump of %g, rmn %d: L1(rho) %.2e L1(en) %.2e" % (jump, rmn, *e))
+    assert max(e) < 1e-6
+
+
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+@pytest.mark.parametrize("odr", [1, 2, 3])
+def test_mixed_across_units_at_lower_orders(odr, rmn):
+    """test_mixed_across_units at ODR 1 to 3: each order's error stays at the
+    size it has in the first units."""
+    from qasmhd_amd import capi, problems
+    p = problems.turbulence2d(n=32, seed=3)
+    with capi.solver_for(p) as s:
+        s.upload(p.state)
+        dt = s.cfl_dt()
+    I = (slice(4, -4), slice(4, -4))
+    for k in (0, 4, 8, 11):
+        q = p.copy()
+        f = 2.0 ** k
+        q.state[1:7] *= f
+        q.state[7] *= f * f
+        out = []
+        for precision in (0, 1):
+            with capi.solver_for(q, rmn=rmn, odr=odr, precision=precision) as s:
+                s.upload(q.state)
+                s.run(4, flg=0, dt=dt / f, history=False)
+                out.append(s.download())
+        e = [l1rel(out[1][m][I], out[0][m][I]) for m in (0, 7)]
+        _say("mixed vs fp64, odr %d, rmn %d, speeds x 2^%d: L1(rho) %.2e L1(en) %.2e" % (odr, rmn, k, *e))
+        assert max(e) < 1e-6
+
+
 def test_mixed_l1_error_vs_oracle(oracle):
     """The mixed path's L1 error measured against the oracle itself (the
     CPU restatement of the reference) rather than through the FP64 HIP
