@@ -136,7 +136,7 @@ struct Hlld {
     }
     x[14] = r.in(-1.0, 1.0);
   }
-  static void fwd(const double* x, double* y) { qas::flux_hlld_family<double>(false, x, x + 7, x[14], gam, 0.0, 0.0, y); }
+  static void fwd(const double* x, double* y) { qas::flux_hlld_family<qas::PlainOps>(false, x, x + 7, x[14], gam, 0.0, 0.0, y); }
   static void adj(const double* x, const double* g, double* gx)
   {
     qas::hlld_adj(x, x + 7, x[14], gam, g, gx, gx + 7, gx[14]);
@@ -162,7 +162,7 @@ struct Mlau {
     x[15] = r.in(-1.0, 1.0);
     x[16] = r.in(-1.0, 1.0);
   }
-  static void fwd(const double* x, double* y) { qas::flux_mlau<double>(x, x + 7, x[14], gam, x[15], x[16], y); }
+  static void fwd(const double* x, double* y) { qas::flux_mlau<qas::PlainOps>(x, x + 7, x[14], gam, x[15], x[16], y); }
   static void adj(const double* x, const double* g, double* gx)
   {
     qas::mlau_adj(x, x + 7, x[14], gam, x[15], x[16], g, gx, gx + 7, gx[14], gx[15], gx[16]);
@@ -176,7 +176,7 @@ struct Lhlld {
   static void sample(Rng& r, double* x) { Mlau::sample(r, x); }
   static void fwd(const double* x, double* y)
   {
-    qas::flux_hlld_family<double>(true, x, x + 7, x[14], gam, x[15], x[16], y);
+    qas::flux_hlld_family<qas::PlainOps>(true, x, x + 7, x[14], gam, x[15], x[16], y);
   }
   static void adj(const double* x, const double* g, double* gx)
   {

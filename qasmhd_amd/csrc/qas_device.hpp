@@ -94,90 +94,105 @@ QAS_HD T div_3p2(T x)
   return x / T(N);
 }
 
-// 1 / x, a / x and sqrt(x) of the point functions: FP64 on the device without
-// the IEEE sequences' operand scaling.  The scaling serves operands near the
-// ends of the exponent range; the estimate, refinement and last residual step
-// are the same, and the fix-up instruction (the class select of the root)
-// gives zeros, infinities and NaN their IEEE results.  Same bits as the
-// operators for operands and results in [2^-960, 2^1000] and for zero,
-// infinite and NaN operands.  inv 7 instructions against 11, a second quotient by
-// the same x (quot with inv_raw(x)) 4 against 11, root 13 against 18; the
-// HLLD flux forms 8 reciprocals, 4 quotients and 5 roots, which take 28 % of
-// its instructions as operators.
-//
+// 1 / x, a / x and sqrt(x) of the point functions on the device without the
+// operators' handling of operands near the ends of the exponent range.
+// FP64: the estimate, refinement and last residual step of the IEEE
+// sequences without their operand scaling, and the fix-up instruction (the
+// class select of the root) for zeros, infinities and NaN: the operators'
+// bits for operands and results in [2^-960, 2^1000] and for zero, infinite
+// and NaN operands.  inv 7 instructions against 11, a second quotient by the
+// same x (quot with raw(x)) 4 against 11, root 13 against 18; the HLLD flux
+// forms 8 reciprocals, 4 quotients and 5 roots, which take 28 % of its
+// instructions as operators.
 // FP32 (the mixed path, built with the fast FP32 division and root): the
 // estimates v_rcp_f32 and v_sqrt_f32 themselves (1 ulp), which that division
-// and root wrap in exponent arithmetic for operands below 2^-96 or above
-// 2^126; the same bits between.  One instruction each against 4 to 6: 230 of
-// 1830 per wavefront of the MLAU y sweep.
-template <typename T>
-QAS_HD T inv_raw(T x)
-{
+// and root wrap in exponent arithmetic; the same bits for operands and
+// results in [2^-126, 2^126], but a reciprocal below and the root of a
+// denormal are 0.  One instruction each against 4 to 6: 230 of 1830 per
+// wavefront of the MLAU y sweep.
+struct FastOps {
+  template <typename T>
+  static QAS_HD T raw(T x)
+  {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_rcpf(x);
+    if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_rcpf(x);
 #endif
-  if constexpr (std::is_same<T, double>::value) return rcp_inrange(x);
-  else return T(1.0) / x;
-}
-
-template <typename T>
-QAS_HD T inv(T x)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_rcpf(x);
-  if constexpr (std::is_same<T, double>::value) return __builtin_amdgcn_div_fixup(rcp_inrange(x), x, 1.0);
-#endif
-  return T(1.0) / x;
-}
-
-// a / x with rx = inv_raw(x)
-template <typename T>
-QAS_HD T quot(T a, T x, T rx)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (std::is_same<T, float>::value) return a * rx;
-  if constexpr (std::is_same<T, double>::value) {
-    const double q = a * rx;
-    return __builtin_amdgcn_div_fixup(fma(fma(-x, q, a), rx, q), x, a);
+    if constexpr (std::is_same<T, double>::value) return rcp_inrange(x);
+    else return T(1.0) / x;
   }
-#endif
-  (void)rx;
-  return a / x;
-}
-
-// a / x, and 0.5 / x (an exact factor)
-template <typename T>
-QAS_HD T ratio(T a, T x)
-{
-  if constexpr (std::is_floating_point<T>::value) return quot(a, x, inv_raw(x));
-  else return a / x;
-}
-
-template <typename T>
-QAS_HD T half_inv(T x)
-{
-  if constexpr (std::is_floating_point<T>::value) return T(0.5) * inv(x);
-  else return T(0.5) / x;
-}
-
-template <typename T>
-QAS_HD T root(T x)
-{
+  template <typename T>
+  static QAS_HD T inv(T x)
+  {
 #if defined(__HIP_DEVICE_COMPILE__)
-  if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_sqrtf(x);
-  if constexpr (std::is_same<T, double>::value) {
-    const double r = __builtin_amdgcn_rsq(x);
-    double g = x * r, h = 0.5 * r;
-    const double e = fma(-h, g, 0.5);
-    g = fma(g, e, g);
-    h = fma(h, e, h);
-    g = fma(fma(-g, g, x), h, g);
-    g = fma(fma(-g, g, x), h, g);
-    return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0 and +inf are their own roots
-  }
+    if constexpr (std::is_same<T, double>::value) return __builtin_amdgcn_div_fixup(rcp_inrange(x), x, 1.0);
 #endif
-  return dsqrt(x);
-}
+    return raw(x);
+  }
+  // a / x with rx = raw(x)
+  template <typename T>
+  static QAS_HD T quot(T a, T x, T rx)
+  {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (std::is_same<T, float>::value) return a * rx;
+    if constexpr (std::is_same<T, double>::value) {
+      const double q = a * rx;
+      return __builtin_amdgcn_div_fixup(fma(fma(-x, q, a), rx, q), x, a);
+    }
+#endif
+    (void)rx;
+    return a / x;
+  }
+  template <typename T>
+  static QAS_HD T ratio(T a, T x)
+  {
+    if constexpr (std::is_floating_point<T>::value) return quot(a, x, raw(x));
+    else return a / x;
+  }
+  template <typename T>
+  static QAS_HD T root(T x)
+  {
+#if defined(__HIP_DEVICE_COMPILE__)
+    if constexpr (std::is_same<T, float>::value) return __builtin_amdgcn_sqrtf(x);
+    if constexpr (std::is_same<T, double>::value) {
+      const double r = __builtin_amdgcn_rsq(x);
+      double g = x * r, h = 0.5 * r;
+      const double e = fma(-h, g, 0.5);
+      g = fma(g, e, g);
+      h = fma(h, e, h);
+      g = fma(fma(-g, g, x), h, g);
+      g = fma(fma(-g, g, x), h, g);
+      return __builtin_amdgcn_class(x, 0x260) ? x : g;  // +-0 and +inf are their own roots
+    }
+#endif
+    return dsqrt(x);
+  }
+};
+
+// the operators, for operands of any size
+struct PlainOps {
+  template <typename T> static QAS_HD T raw(T x) { return T(1.0) / x; }
+  template <typename T> static QAS_HD T inv(T x) { return T(1.0) / x; }
+  template <typename T> static QAS_HD T quot(T a, T x, T) { return a / x; }
+  template <typename T> static QAS_HD T ratio(T a, T x) { return a / x; }
+  template <typename T> static QAS_HD T root(T x) { return dsqrt(x); }
+};
+
+// Whether the magnitudes add()ed so far all lie in [2^-25, 2^25): two integer
+// instructions per value on the exponent bits.  A point function whose
+// densities, pressures and energies pass has all its speeds, masses, products
+// and roots' arguments in the FP32 range of FastOps; a wavefront with a lane
+// outside() (a uniform value) takes PlainOps.  The tests and their branches
+// take 0.5 to 1.2 % of a run (MLAU at 2048^2, HLLD at 200^3).
+struct ModerateFloats {
+  static constexpr unsigned LOW = (127u - 25u) << 24, SPAN = 50u << 24;
+  unsigned top = 0;
+  __device__ __forceinline__ void add(float x)
+  {
+    const unsigned k = ((unsigned)__float_as_int(x) << 1) - LOW;  // exponent and significand, the sign shifted out
+    top = top > k ? top : k;
+  }
+  __device__ __forceinline__ bool outside() const { return __any(top >= SPAN) != 0; }
+};
 
 // ------------------------------------------------------------------ 1-D interpolation
 // f[0..4] = stencil i-2..i+2; fl = left state at i+1/2, fr = right state at i-1/2.
@@ -214,7 +229,7 @@ QAS_HD T minmod(T a, T b)
 
 // The weights and face values of WCNS-4 (common_interp.c:102-150) from
 // the three denominators d_k = IS_k^2 + eps; IN_RANGE takes the reciprocals
-// with inv_raw (the caller checked the range), else 1.0 / x.
+// with FastOps::raw (the caller checked the range), else 1.0 / x.
 // Returns 8 fl and 8 fr: the face values without their factor 1/8, which is
 // exact and which lrstate folds into its coefficients.  Products with powers
 // of two go into the following add (fma2, same rounding), and 6 f = 2 (3 f).
@@ -222,7 +237,7 @@ template <bool IN_RANGE, typename T>
 QAS_HD void wcns4_weights(const T* f, T d0, T d1, T d2, T& fl8, T& fr8)
 {
   auto inv = [](T x) -> T {
-    if constexpr (IN_RANGE) return inv_raw(x);
+    if constexpr (IN_RANGE) return FastOps::raw(x);
     else return T(1.0) / x;
   };
   const T s0 = inv(d0);
@@ -303,25 +318,21 @@ QAS_HD void interp5(const T* f, T& fl, T& fr)
       w1 = T(1.0) - w0;
       fr = T(0.5) * (w1 * (-f[3] + T(3.0) * f[2]) + w0 * (f[2] + f[1]));
     };
-    if constexpr (INRANGE && std::is_floating_point<T>::value) {
-      // t <= 4 max(s0, s1), and eps is 2^-133 (FP32 2^-100): s0, s1 <= 2^700
-      // keep the denominators and the weight sums below 2^837, where the
-      // reciprocal has its precision.  In FP32 2^120 keeps the first
-      // denominators in the range of v_rcp_f32, which gives 0 from 2^126 on;
-      // the weight sums may be t / eps (beside a flat pair, s0 = 0: past 2^126
-      // from a difference of 1.07e4 on, past FP32 from 1.84e4 on) and are
-      // held below 2^126.  NaN fails the test.
-      constexpr T top = sizeof(T) == 8 ? T(0x1p700) : T(0x1p120);
-      bool in = (s0 <= top) & (s1 <= top);
+    if constexpr (std::is_same<T, float>::value) {
+      // v_rcp_f32 gives 0 from 2^126 on: the first denominators are tested
+      // (2^120); the weight sums may be t / eps (beside a flat pair, s0 = 0:
+      // past 2^126 from a difference of 1.07e4 on, past FP32 from 1.84e4 on)
+      // and are held below 2^126.  NaN fails the test.
+      bool in = (s0 <= T(0x1p120)) & (s1 <= T(0x1p120));
 #if defined(__HIP_DEVICE_COMPILE__)
-      if constexpr (sizeof(T) == 4) in = __all(in) != 0;
+      in = __all(in) != 0;
 #endif
-      if (in) {
-        face([](T x, T y) { return ratio(x, y); });
+      if (!in) {
+        face([](T x, T y) { return x / y; });
         return;
       }
     }
-    face([](T x, T y) { return x / y; });
+    face([](T x, T y) { return FastOps::ratio(x, y); });
   } else {  // WCNS4
     const T eps = wcns_eps<T>();
     const T c13 = T(13. / 12.);
@@ -440,24 +451,42 @@ QAS_HD void lrstate_of(const S& s, T bn, T gam, T (&vl)[7], T (&vr)[7], int* fbc
   const bool anyf = MODE != 2;
 #endif
   // shared eigen quantities (mhd_eigen_mi / mhd_eigen_ae)
-  const T iro = inv(ro0);
-  const T cs2 = gam * pr0 * iro;
-  const T ca2 = bn * bn * iro;
-  const T ct2 = (bt0 * bt0 + bu0 * bu0) * iro;
-  const T cb2 = cs2 + ca2 + ct2;
-  const T cf2 = T(0.5) * (cb2 + root(dabs(fma2(T(-4.0), cs2 * ca2, cb2 * cb2))));
-  T rcf = T(0.0), icf2h = T(0.0), ircfh = T(0.0);
-  if (MODE != 2 && anyf) {
-    const T cf = root(cf2);
-    rcf = ro0 * cf;
+  T cf2, rcf = T(0.0), icf2, icf2h = T(0.0), ircfh = T(0.0), sro, isroh;
+  auto eigen = [&](auto o) {
+    const T iro = o.inv(ro0);
+    const T cs2 = gam * pr0 * iro;
+    const T ca2 = bn * bn * iro;
+    const T ct2 = (bt0 * bt0 + bu0 * bu0) * iro;
+    const T cb2 = cs2 + ca2 + ct2;
+    cf2 = T(0.5) * (cb2 + o.root(dabs(fma2(T(-4.0), cs2 * ca2, cb2 * cb2))));
+    if (MODE != 2 && anyf) {
+      const T cf = o.root(cf2);
+      rcf = ro0 * cf;
+    }
+    sro = o.root(ro0);
+    if constexpr (std::is_floating_point<T>::value) isroh = T(0.5) * o.inv(sro);
+    else isroh = T(0.5) / sro;
+    icf2 = o.inv(cf2);
+    if (MODE != 2 && anyf) {
+      icf2h = T(0.5) * icf2;
+      if constexpr (std::is_floating_point<T>::value) ircfh = T(0.5) * o.inv(rcf);
+      else ircfh = T(0.5) / rcf;
+    }
+  };
+#if defined(__HIP_DEVICE_COMPILE__)
+  bool plain = false;
+  if constexpr (std::is_same<T, float>::value) {
+    ModerateFloats m;
+    m.add(ro0);
+    m.add(pr0);
+    m.add(pr0 + (bn * bn + bt0 * bt0 + bu0 * bu0));
+    plain = m.outside();
   }
-  const T sro = root(ro0);
-  const T isroh = half_inv(sro);
-  const T icf2 = inv(cf2);
-  if (MODE != 2 && anyf) {
-    icf2h = T(0.5) * icf2;
-    ircfh = half_inv(rcf);
-  }
+  if (__builtin_expect(plain, 0)) eigen(PlainOps{});
+  else eigen(FastOps{});
+#else
+  eigen(PlainOps{});
+#endif
   const T byh = T(0.5) * bt0;
   const T bzh = T(0.5) * bu0;
 
@@ -645,23 +674,23 @@ QAS_HD bool positive_sum(T vn, T b, T r)
   return vn + b / r > T(0);
 }
 
-template <typename T>
+template <typename O, typename T>
 QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, T gamma,
                                                  T dv0, T dv1, T* F)
 {
   const T FL_EPS = T(QAS_FL_EPS);
   const T rol = L[0], vnl = L[1], vtl = L[2], vul = L[3], btl = L[4], bul = L[5], prl = L[6];
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
-  const T gammam1i = inv(gamma - T(1.0));
+  const T gammam1i = O::inv(gamma - T(1.0));
   const T bnc2 = bnc * bnc;
   const T sgn = (bnc > T(0)) ? T(1.0) : T(-1.0);
-  const T roli = inv(rol);
+  const T roli = O::inv(rol);
   const T b2l = btl * btl + bul * bul;  // twice the transverse magnetic pressure
   const T ptl = fma2(T(0.5), b2l, prl);
   const T vl2 = vnl * vnl + vtl * vtl + vul * vul;
   const T enl = fma2(T(0.5), rol * vl2, fma2(T(0.5), b2l, gammam1i * prl));
   const T vbl = vtl * btl + vul * bul;
-  const T rori = inv(ror);
+  const T rori = O::inv(ror);
   const T b2r = btr * btr + bur * bur;
   const T ptr = fma2(T(0.5), b2r, prr);
   const T vr2 = vnr * vnr + vtr * vtr + vur * vur;
@@ -674,32 +703,32 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   const T cbl2 = cl2 + cal2 + b2l * roli;
   const T cbr2 = cr2 + car2 + b2r * rori;
   // twice the squared fast speeds
-  const T cfl2 = cbl2 + root(dabs(fma2(T(-4.0), cl2 * cal2, cbl2 * cbl2)));
-  const T cfr2 = cbr2 + root(dabs(fma2(T(-4.0), cr2 * car2, cbr2 * cbr2)));
+  const T cfl2 = cbl2 + O::root(dabs(fma2(T(-4.0), cl2 * cal2, cbl2 * cbl2)));
+  const T cfr2 = cbr2 + O::root(dabs(fma2(T(-4.0), cr2 * car2, cbr2 * cbr2)));
   T ccl2 = T(0), ccr2 = T(0);  // twice the squared speeds with |v| for the sound speed
   if (lowdiss) {
     const T cbl2c = vl2 + cal2 + b2l * roli;
     const T cbr2c = vr2 + car2 + b2r * rori;
-    ccl2 = cbl2c + root(dabs(fma2(T(-4.0), vl2 * cal2, cbl2c * cbl2c)));
-    ccr2 = cbr2c + root(dabs(fma2(T(-4.0), vr2 * car2, cbr2c * cbr2c)));
+    ccl2 = cbl2c + O::root(dabs(fma2(T(-4.0), vl2 * cal2, cbl2c * cbl2c)));
+    ccr2 = cbr2c + O::root(dabs(fma2(T(-4.0), vr2 * car2, cbr2c * cbr2c)));
   }
   // the larger of the two fast speeds; a correctly rounded root is monotonic,
   // so the root of the larger square is the larger root
-  const T cmax = root(T(0.5) * tmax(cfl2, cfr2));
+  const T cmax = O::root(T(0.5) * tmax(cfl2, cfr2));
   const T sl = tmin(T(0.0), tmin(vnl, vnr) - cmax);
   const T sr = tmax(T(0.0), tmax(vnl, vnr) + cmax);
   const T slvl = sl - vnl;
   const T srvr = sr - vnr;
   const T rslvl = rol * slvl;
   const T rsrvr = ror * srvr;
-  const T drsvi = inv(rsrvr - rslvl);
+  const T drsvi = O::inv(rsrvr - rslvl);
   T vnc, ptc;
   if (lowdiss) {
-    T theta = tmin(T(1.0), ratio(cmax - tmin(dv0, T(0.0)), cmax - tmin(dv1, T(0.0))));
+    T theta = tmin(T(1.0), O::ratio(cmax - tmin(dv0, T(0.0)), cmax - tmin(dv1, T(0.0))));
     theta *= theta;
     theta *= theta;
     vnc = (rsrvr * vnr - rslvl * vnl - theta * (ptr - ptl)) * drsvi;
-    const T mcc = tmin(T(1.0), ratio(root(T(0.5) * tmax(ccl2, ccr2)), cmax));
+    const T mcc = tmin(T(1.0), O::ratio(O::root(T(0.5) * tmax(ccl2, ccr2)), cmax));
     ptc = (rsrvr * ptl - rslvl * ptr + (mcc * (T(2.0) - mcc)) * rsrvr * rslvl * (vnr - vnl)) * drsvi;
   } else {
     vnc = (rsrvr * vnr - rslvl * vnl - ptr + ptl) * drsvi;
@@ -707,16 +736,16 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   }
   const T slvc = sl - vnc;
   const T srvc = sr - vnc;
-  const T slvci = inv_raw(slvc);
-  const T srvci = inv_raw(srvc);
-  const T ro2l = quot(rslvl, slvc, slvci);
-  const T ro2r = quot(rsrvr, srvc, srvci);
+  const T slvci = O::raw(slvc);
+  const T srvci = O::raw(srvc);
+  const T ro2l = O::quot(rslvl, slvc, slvci);
+  const T ro2r = O::quot(rsrvr, srvc, srvci);
   const T rhdl = rslvl * slvc - bnc2;
   const T rhdr = rsrvr * srvc - bnc2;
   T vt2l = vtl, vu2l = vul, bt2l = btl, bu2l = bul;
   T vt2r = vtr, vu2r = vur, bt2r = btr, bu2r = bur;
   if (dabs(rhdl) > FL_EPS) {
-    const T rhdli = inv(rhdl);
+    const T rhdli = O::inv(rhdl);
     const T rhnvl = (vnl - vnc) * bnc;
     const T rhnbl = rslvl * slvl - bnc2;
     vt2l = vtl + rhnvl * rhdli * btl;
@@ -725,7 +754,7 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
     bu2l = rhnbl * rhdli * bul;
   }
   if (dabs(rhdr) > FL_EPS) {
-    const T rhdri = inv(rhdr);
+    const T rhdri = O::inv(rhdr);
     const T rhnvr = (vnr - vnc) * bnc;
     const T rhnbr = rsrvr * srvr - bnc2;
     vt2r = vtr + rhnvr * rhdri * btr;
@@ -735,11 +764,11 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   }
   const T vb2l = vt2l * bt2l + vu2l * bu2l;
   const T vb2r = vt2r * bt2r + vu2r * bu2r;
-  const T en2l = quot(slvl * enl - ptl * vnl + ptc * vnc + bnc * (vbl - vb2l), slvc, slvci);
-  const T en2r = quot(srvr * enr - ptr * vnr + ptc * vnc + bnc * (vbr - vb2r), srvc, srvci);
-  const T rro2l = root(ro2l);
-  const T rro2r = root(ro2r);
-  const T rro2i = inv(rro2r + rro2l);
+  const T en2l = O::quot(slvl * enl - ptl * vnl + ptc * vnc + bnc * (vbl - vb2l), slvc, slvci);
+  const T en2r = O::quot(srvr * enr - ptr * vnr + ptc * vnc + bnc * (vbr - vb2r), srvc, srvci);
+  const T rro2l = O::root(ro2l);
+  const T rro2r = O::root(ro2r);
+  const T rro2i = O::inv(rro2r + rro2l);
   const T vt3m = fma2(sgn, bt2r - bt2l, rro2r * vt2r + rro2l * vt2l) * rro2i;
   const T vu3m = fma2(sgn, bu2r - bu2l, rro2r * vu2r + rro2l * vu2l) * rro2i;
   const T bt3m = fma2(sgn, rro2r * rro2l * (vt2r - vt2l), rro2l * bt2r + rro2r * bt2l) * rro2i;
@@ -768,23 +797,23 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   F[6] = (enu + ptc) * vnc - bnc * (vtu * btu + vuu * buu);
 }
 
-template <typename T>
+template <typename O, typename T>
 QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F)
 {
   const T FL_EPS = T(QAS_FL_EPS);
   const T rol = L[0], vnl = L[1], vtl = L[2], vul = L[3], btl = L[4], bul = L[5], prl = L[6];
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
-  const T gammam1i = inv(gamma - T(1.0));
+  const T gammam1i = O::inv(gamma - T(1.0));
   const T bnc2 = bnc * bnc;
   const T sgn = (bnc > T(0)) ? T(1.0) : T(-1.0);
   const T bnca = sgn * bnc;
-  const T roli = inv(rol);
+  const T roli = O::inv(rol);
   const T vl2 = vnl * vnl + vtl * vtl + vul * vul;
   const T pml = T(0.5) * (btl * btl + bul * bul);
   const T ptl = prl + pml;
   const T enl = gammam1i * prl + pml + T(0.5) * rol * vl2;
   const T hnl = (enl + ptl) * roli;
-  const T rori = inv(ror);
+  const T rori = O::inv(ror);
   const T vr2 = vnr * vnr + vtr * vtr + vur * vur;
   const T pmr = T(0.5) * (btr * btr + bur * bur);
   const T ptr = prr + pmr;
@@ -796,22 +825,22 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T car2 = bnc2 * rori;
   T cbl2 = cl2 + cal2 + T(2.0) * pml * roli;
   T cbr2 = cr2 + car2 + T(2.0) * pmr * rori;
-  const T cfl2 = T(0.5) * (cbl2 + root(dabs(cbl2 * cbl2 - T(4.0) * cl2 * cal2)));
-  const T cfr2 = T(0.5) * (cbr2 + root(dabs(cbr2 * cbr2 - T(4.0) * cr2 * car2)));
+  const T cfl2 = T(0.5) * (cbl2 + O::root(dabs(cbl2 * cbl2 - T(4.0) * cl2 * cal2)));
+  const T cfr2 = T(0.5) * (cbr2 + O::root(dabs(cbr2 * cbr2 - T(4.0) * cr2 * car2)));
   cbl2 = vl2 + cal2 + T(2.0) * pml * roli;
   cbr2 = vr2 + car2 + T(2.0) * pmr * rori;
-  const T ccl2 = T(0.5) * (cbl2 + root(dabs(cbl2 * cbl2 - T(4.0) * vl2 * cal2)));
-  const T ccr2 = T(0.5) * (cbr2 + root(dabs(cbr2 * cbr2 - T(4.0) * vr2 * car2)));
-  const T cmax = root(tmax(cfl2, cfr2));
+  const T ccl2 = T(0.5) * (cbl2 + O::root(dabs(cbl2 * cbl2 - T(4.0) * vl2 * cal2)));
+  const T ccr2 = T(0.5) * (cbr2 + O::root(dabs(cbr2 * cbr2 - T(4.0) * vr2 * car2)));
+  const T cmax = O::root(tmax(cfl2, cfr2));
   const T cfn = cmax;
-  const T cfni = inv(cfn);
+  const T cfni = O::inv(cfn);
   const T sl = tmin(T(0.0), tmin(vnl, vnr) - cmax);
   const T sr = tmax(T(0.0), tmax(vnl, vnr) + cmax);
   const T mal = vnl * cfni;
   const T mar = vnr * cfni;
   const T snl = (mal > T(0)) ? T(1.0) : T(-1.0);
   const T snr = (mar > T(0)) ? T(1.0) : T(-1.0);
-  T theta = tmin(T(1.0), ratio(cfn - tmin(dv0, T(0.0)), cfn - tmin(dv1, T(0.0))));
+  T theta = tmin(T(1.0), O::ratio(cfn - tmin(dv0, T(0.0)), cfn - tmin(dv1, T(0.0))));
   theta *= theta;
   theta *= theta;
   const T alpha = T(0.1875);
@@ -837,7 +866,7 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   }
   const T mnc = ffl + ffr;
   T mflux = mnc * cfn;
-  mflux -= ratio(tmax(T(1.0) - dabs(mnc), T(0.0)) * theta * cfni * (ptr - ptl), rol + ror);
+  mflux -= O::ratio(tmax(T(1.0) - dabs(mnc), T(0.0)) * theta * cfni * (ptr - ptl), rol + ror);
   const T dir = (mflux > T(0)) ? T(1.0) : T(-1.0);
   const T dirl = T(0.5) * (T(1.0) + dir);
   const T dirr = T(1.0) - dirl;
@@ -845,31 +874,31 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T mfl = mflux * dirl;
   const T mfr = mflux - mfl;
   T ptot = bfl * ptl + bfr * ptr;
-  const T cfmod = root(tmax(ccl2, ccr2));
+  const T cfmod = O::root(tmax(ccl2, ccr2));
   ptot -= T(0.25) * bfl * bfr * (rol + ror) * cfmod * (vnr - vnl);
   ptot -= T(0.5) * (T(1.0) - cfmod * cfni) * (bfl + bfr - T(1.0)) * (ptl + ptr);
   const T slvl = sl - vnl;
   const T srvr = sr - vnr;
   const T snc = dirl * sl + dirr * sr;
   const T vndnm = mflux + dirl * rol * slvl + dirr * ror * srvr;
-  const T vnc = ((dabs(vndnm) > FL_EPS) && (snc != T(0))) ? ratio(mflux * snc, vndnm) : (dirl * vnl + dirr * vnr);
+  const T vnc = ((dabs(vndnm) > FL_EPS) && (snc != T(0))) ? O::ratio(mflux * snc, vndnm) : (dirl * vnl + dirr * vnr);
   const T slvc = sl - vnc;
   const T srvc = sr - vnc;
-  const T slvci = inv(slvc);
-  const T srvci = inv(srvc);
+  const T slvci = O::inv(slvc);
+  const T srvci = O::inv(srvc);
   const T rhdl = rol * slvl * slvc - bnc2;
   const T rhdr = ror * srvr * srvc - bnc2;
   T dvtl = T(0.0), dvul = T(0.0), dbtl = T(0.0), dbul = T(0.0);
   T dvtr = T(0.0), dvur = T(0.0), dbtr = T(0.0), dbur = T(0.0);
   if (dabs(rhdl) > FL_EPS) {
-    const T q = ratio(vnc - vnl, rhdl);
+    const T q = O::ratio(vnc - vnl, rhdl);
     dvtl = -bnc * btl * q;
     dvul = -bnc * bul * q;
     dbtl = bnc2 * btl * q * slvci;
     dbul = bnc2 * bul * q * slvci;
   }
   if (dabs(rhdr) > FL_EPS) {
-    const T q = ratio(vnc - vnr, rhdr);
+    const T q = O::ratio(vnc - vnr, rhdr);
     dvtr = -bnc * btr * q;
     dvur = -bnc * bur * q;
     dbtr = bnc2 * btr * q * srvci;
@@ -878,24 +907,24 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   const T cmpl = slvl * slvci;
   const T cmpr = srvr * srvci;
   const T ro2l = rol * cmpl;
-  const T srol = root(ro2l);
+  const T srol = O::root(ro2l);
   const T vt2l = dvtl + vtl;
   const T vu2l = dvul + vul;
   const T bt2l = dbtl + btl * cmpl;
   const T bu2l = dbul + bul * cmpl;
   const T ro2r = ror * cmpr;
-  const T sror = root(ro2r);
+  const T sror = O::root(ro2r);
   const T vt2r = dvtr + vtr;
   const T vu2r = dvur + vur;
   const T bt2r = dbtr + btr * cmpr;
   const T bu2r = dbur + bur * cmpr;
-  const T sroi = inv(srol + sror);
+  const T sroi = O::inv(srol + sror);
   const T srollri = srol * sroi;
   const T srorlri = sror * sroi;
   const T bnflb = sgn * tmin(tmax(T(0.0), srollri * (bnca + sror * vnc)), bnca);
   const T bnfrb = sgn * tmin(tmax(T(0.0), srorlri * (bnca - srol * vnc)), bnca);
-  const T bnflv = sgn * tmin(tmax(T(0.0), srorlri * (bnca + ratio(mflux, sror))), bnca);
-  const T bnfrv = sgn * tmin(tmax(T(0.0), srollri * (bnca - ratio(mflux, srol))), bnca);
+  const T bnflv = sgn * tmin(tmax(T(0.0), srorlri * (bnca + O::ratio(mflux, sror))), bnca);
+  const T bnfrv = sgn * tmin(tmax(T(0.0), srollri * (bnca - O::ratio(mflux, srol))), bnca);
   const T bnsrv = tmax(bnca - dir * vnc * (dirl * srol + dirr * sror), T(0.0));
   const T ccb = sroi * bnsrv;
   const T ccv = srol * sror * ccb;
@@ -918,7 +947,9 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   rv2b2 *= rv2b2;
   T vb3 = T(0.0);
   if (rv2b2 > FL_EPS * FL_EPS) {
-    vb3 = ratio(+(fmt * vnc + fbt * bnc) * (fmt * bnc + fbt * mflux) +
+    // (in FP32 a denominator of eight factors may leave the reciprocal's range)
+    using V = typename std::conditional<std::is_same<T, float>::value, PlainOps, O>::type;
+    vb3 = V::ratio(+(fmt * vnc + fbt * bnc) * (fmt * bnc + fbt * mflux) +
                     (fmu * vnc + fbu * bnc) * (fmu * bnc + fbu * mflux),
                 rv2b2);
   }
@@ -932,7 +963,7 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   F[6] = mfl * hnl + mfr * hnr - bnvb;
 }
 
-template <typename T>
+template <typename O, typename T>
 QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
 {
   const T FL_EPS = T(QAS_FL_EPS);
@@ -940,16 +971,16 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
   const T gammam1 = gamma - T(1.0);
   const T gammam2 = gamma - T(2.0);
-  const T gammam1i = inv(gammam1);
-  const T roli = inv(rol);
-  const T rori = inv(ror);
-  const T rrol = root(rol);
-  const T rror = root(ror);
-  const T rroi = inv(rrol + rror);
+  const T gammam1i = O::inv(gammam1);
+  const T roli = O::inv(rol);
+  const T rori = O::inv(ror);
+  const T rrol = O::root(rol);
+  const T rror = O::root(ror);
+  const T rroi = O::inv(rrol + rror);
   const T robar = rrol * rror;
-  const T robari = inv(robar);
-  const T rrobar = root(robar);
-  const T rrobai = root(robari);
+  const T robari = O::inv(robar);
+  const T rrobar = O::root(robar);
+  const T rrobai = O::root(robari);
   const T vnbar = (rrol * vnl + rror * vnr) * rroi;
   const T vtbar = (rrol * vtl + rror * vtr) * rroi;
   const T vubar = (rrol * vul + rror * vur) * rroi;
@@ -971,28 +1002,28 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T a2 = (gammam1 * (+hbar - v2b - db2) - gammam2 * bb2 * robari);
   const T ca2 = bnbar * bnbar * robari;
   const T cb2 = (btbar * btbar + bubar * bubar) * robari;
-  const T cf2 = T(0.5) * (a2 + root(cb2 * (a2 + c2 + ca2) + (c2 - ca2) * (c2 - ca2)));
-  const T cs2 = ratio(c2 * ca2, cf2);
-  const T cf = root(cf2);
-  const T cs = root(cs2);
-  const T ca = root(ca2);
-  const T c = root(c2);
-  const T cfi = inv(cf);
+  const T cf2 = T(0.5) * (a2 + O::root(cb2 * (a2 + c2 + ca2) + (c2 - ca2) * (c2 - ca2)));
+  const T cs2 = O::ratio(c2 * ca2, cf2);
+  const T cf = O::root(cf2);
+  const T cs = O::root(cs2);
+  const T ca = O::root(ca2);
+  const T c = O::root(c2);
+  const T cfi = O::inv(cf);
   const T sgr1 = btbar * btbar + bubar * bubar - FL_EPS;
   const T sf11 = (sgr1 > T(0)) ? T(1.0) : T(0.0);
   const T sf21 = T(1.0) - sf11;
-  const T beti = inv(root(btbar * btbar + bubar * bubar + sf21));
-  const T bett = sf11 * btbar * beti + sf21 * root(T(0.5));
-  const T betu = sf11 * bubar * beti + sf21 * root(T(0.5));
+  const T beti = O::inv(O::root(btbar * btbar + bubar * bubar + sf21));
+  const T bett = sf11 * btbar * beti + sf21 * O::root(T(0.5));
+  const T betu = sf11 * bubar * beti + sf21 * O::root(T(0.5));
   const T sgr2 = (btbar * btbar + bubar * bubar) * robari + dabs(ca2 - c2) - FL_EPS;
   const T sf12 = (sgr2 > T(0)) ? T(1.0) : T(0.0);
   const T sf22 = T(1.0) - sf12;
   const T cfca = tmax(T(0.0), cf2 - ca2);
   const T cfcs = tmax(T(0.0), cf2 - cs2);
   const T cfa = tmax(T(0.0), cf2 - c2);
-  const T alpi = inv(root(cfcs + sf22));
-  const T alpf = sf12 * root(cfca) * alpi + sf22;
-  const T alps = sf12 * root(cfa) * alpi;
+  const T alpi = O::inv(O::root(cfcs + sf22));
+  const T alpf = sf12 * O::root(cfca) * alpi + sf22;
+  const T alps = sf12 * O::root(cfa) * alpi;
   const T eeps = T(0.0);
   const T evpf = tmax(dabs(vnbar + cf), eeps);
   const T evmf = tmax(dabs(vnbar - cf), eeps);
@@ -1021,8 +1052,8 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T q12 = alps * cs;
   const T q21 = -alps * ca * sgn;
   const T q22 = alpf * c * sgn;
-  const T detpi = inv(p11 * p22 - p12 * p21);
-  const T detqi = inv(q11 * q22 - q12 * q21);
+  const T detpi = O::inv(p11 * p22 - p12 * p21);
+  const T detqi = O::inv(q11 * q22 - q12 * q21);
   const T wvpf = T(0.5) * ((p22 * t1 - p12 * t2) * detpi + (q22 * s1 - q12 * s2) * detqi);
   const T wvmf = T(0.5) * ((p22 * t1 - p12 * t2) * detpi - (q22 * s1 - q12 * s2) * detqi);
   const T wvps = T(0.5) * ((-p21 * t1 + p11 * t2) * detpi + (-q21 * s1 + q11 * s2) * detqi);
@@ -1112,14 +1143,40 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
                    ama * rvmaen - a00 * rv00en);
 }
 
+template <int RMN, typename O, typename T>
+QAS_HD void riemann_of(const T* L, const T* R, T bn, T gam, T dv0, T dv1, T* F)
+{
+  if constexpr (RMN == 0) flux_roe<O>(L, R, bn, gam, F);
+  else if constexpr (RMN == 1) flux_hlld_family<O>(false, L, R, bn, gam, dv0, dv1, F);
+  else if constexpr (RMN == 2) flux_hlld_family<O>(true, L, R, bn, gam, dv0, dv1, F);
+  else flux_mlau<O>(L, R, bn, gam, dv0, dv1, F);
+}
+
 // riemann[RMN] (common/mhd_class.hpp:102-105)
 template <int RMN, typename T>
 QAS_HD void riemann(const T* L, const T* R, T bn, T gam, T dv0, T dv1, T* F)
 {
-  if constexpr (RMN == 0) flux_roe(L, R, bn, gam, F);
-  else if constexpr (RMN == 1) flux_hlld_family(false, L, R, bn, gam, dv0, dv1, F);
-  else if constexpr (RMN == 2) flux_hlld_family(true, L, R, bn, gam, dv0, dv1, F);
-  else flux_mlau(L, R, bn, gam, dv0, dv1, F);
+#if defined(__HIP_DEVICE_COMPILE__)
+  if constexpr (std::is_same<T, float>::value) {
+    ModerateFloats m;
+    for (const T* q : {L, R}) {
+      m.add(q[0]);
+      m.add(q[6]);
+      m.add(q[6] + (q[0] * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) + (q[4] * q[4] + q[5] * q[5]) + bn * bn));
+    }
+    if constexpr (RMN >= 2) {
+      m.add(T(1.0) + dabs(dv0));
+      m.add(T(1.0) + dabs(dv1));
+    }
+    if (__builtin_expect(m.outside(), 0)) {
+      riemann_of<RMN, PlainOps>(L, R, bn, gam, dv0, dv1, F);
+      return;
+    }
+  }
+  riemann_of<RMN, FastOps>(L, R, bn, gam, dv0, dv1, F);
+#else
+  riemann_of<RMN, PlainOps>(L, R, bn, gam, dv0, dv1, F);
+#endif
 }
 
 // mhd_cuct_weight from the corner's four cell means and two face means
@@ -1129,14 +1186,14 @@ QAS_HD T cuct_weight(T ro0, T ro1, T ro2, T ro3, T va0, T va1, T va2, T va3, T v
 {
   const T eps = T(1e-12);
   T roc = T(0.25) * (ro0 + ro1 + ro2 + ro3);
-  roc = inv(root(roc));
+  roc = FastOps::inv(FastOps::root(roc));
   T vac = T(0.25) * (va0 + va1 + va2 + va3);
   T vbc = T(0.25) * (vb0 + vb1 + vb2 + vb3);
   const T bac = T(0.5) * (ba1 + ba3);
   const T bbc = T(0.5) * (bb2 + bb3);
   vac = dabs(vac) + dabs(bac * roc);
   vbc = dabs(vbc) + dabs(bbc * roc);
-  return ratio(vac + T(0.5) * eps, vac + vbc + eps);
+  return FastOps::ratio(vac + T(0.5) * eps, vac + vbc + eps);
 }
 
 // rk_updt (common/common_func.h:28-32)

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(WAVE) void k_stage1d(StagePtrs p, Geo g, BcFlags bc
     }
 #pragma unroll
     for (int e = 0; e < 2; e++) {
-      const double iro = inv(u[e][0]);
+      const double iro = FastOps::inv(u[e][0]);
       const double vx = u[e][1] * iro, vy = u[e][2] * iro, vz = u[e][3] * iro;
       const double v2 = vx * vx + vy * vy + vz * vz;
       const double b2 = u[e][4] * u[e][4] + u[e][5] * u[e][5] + u[e][6] * u[e][6];

@@ -56,7 +56,7 @@ __device__ __forceinline__ Prim2d prim2d_cell(const StagePtrs& p, const Geo& g, 
   }
   }
   const double ro = G(p.in[0])[t];
-  const double iro = inv(ro);
+  const double iro = FastOps::inv(ro);
   r.vx = G(p.in[1])[t] * iro;
   r.vy = G(p.in[2])[t] * iro;
   r.vz = G(p.in[3])[t] * iro;
@@ -78,7 +78,7 @@ __device__ __forceinline__ Prim2d prim2d_cell(const StagePtrs& p, const Geo& g, 
 // prim kernel (m * (1/ro)), so the FP64 value is bit-identical to it
 __device__ __forceinline__ double vel(const StagePtrs& p, int comp, long long c)
 {
-  return p.in[1 + comp][c] * inv(p.in[0][c]);
+  return p.in[1 + comp][c] * FastOps::inv(p.in[0][c]);
 }
 
 // ------------------------------------------------------------------ EMF

@@ -20,7 +20,7 @@ template <typename T>
 struct VelOf {
   const double* m;
   const double* ro;
-  __device__ __forceinline__ T operator[](long long q) const { return (T)(m[q] * inv(ro[q])); }
+  __device__ __forceinline__ T operator[](long long q) const { return (T)(m[q] * FastOps::inv(ro[q])); }
 };
 
 // shock sensor dv of mhd2d_solve.cpp:105-125 at (i, j) after its bound():

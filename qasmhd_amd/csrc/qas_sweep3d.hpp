@@ -87,7 +87,7 @@ __device__ __forceinline__ Prim3d prim3d_cell(const StagePtrs& p, const Geo& g, 
     }
   }
   const double ro = p.in[0][t];
-  const double iro = inv(ro);
+  const double iro = FastOps::inv(ro);
   r.vx = p.in[1][t] * iro;
   r.vy = p.in[2][t] * iro;
   r.vz = p.in[3][t] * iro;

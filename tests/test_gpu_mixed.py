@@ -142,6 +142,40 @@ def test_mixed_across_units_at_lower_orders(odr, rmn):
         assert max(e) < 1e-6
 
 
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+@pytest.mark.parametrize("odr", [1, 2, 3])
+def test_mixed_at_small_speeds(odr, rmn):
+    """Units in which the speeds are 2^k and the densities 2^b (pressures stay
+    above the positivity floor): below 2^-31 the squares of the squared speeds
+    are FP32 denormals, which the root estimate takes for 0, so the operators
+    must serve there.  Same error as in the first units; at 2^-33 the
+    denormals keep 9 bits of those squares, which is 1e-3 of a quarter of the
+    squared speed in a dissipation that acts on differences of 1e-4.  (Roe's
+    mean field energy underflows from 2^-32 on.)"""
+    from qasmhd_amd import capi, problems
+    p = problems.turbulence2d(n=32, seed=3)
+    with capi.solver_for(p) as s:
+        s.upload(p.state)
+        dt = s.cfl_dt()
+    I = (slice(4, -4), slice(4, -4))
+    for k, b in ((-10, 20), (-28, 60), (-31, 64)) + (((-33, 70),) if rmn else ()):
+        q = p.copy()
+        f, d = 2.0 ** k, 2.0 ** b
+        q.state[0] *= d
+        q.state[1:4] *= f * d
+        q.state[4:7] *= f * np.sqrt(d)
+        q.state[7] *= f * f * d
+        out = []
+        for precision in (0, 1):
+            with capi.solver_for(q, rmn=rmn, odr=odr, precision=precision) as s:
+                s.upload(q.state)
+                s.run(4, flg=0, dt=dt / f, history=False)
+                out.append(s.download())
+        e = [l1rel(out[1][m][I], out[0][m][I]) for m in (0, 7)]
+        _say("mixed vs fp64, odr %d, rmn %d, speeds 2^%d, densities 2^%d: L1(rho) %.2e L1(en) %.2e" % (odr, rmn, k, b, *e))
+        assert max(e) < 1e-6
+
+
 def test_mixed_l1_error_vs_oracle(oracle):
     """The mixed path's L1 error measured against the oracle itself (the
     CPU restatement of the reference) rather than through the FP64 HIP
