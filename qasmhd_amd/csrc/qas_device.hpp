@@ -800,6 +800,9 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
 template <typename O, typename T>
 QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F)
 {
+  // quotients whose numerator may be of any size (velocities at rest but for
+  // the tail of a perturbation): FP64 would lose quot's residual below 2^-960
+  using V = typename std::conditional<std::is_same<T, double>::value, PlainOps, O>::type;
   const T FL_EPS = T(QAS_FL_EPS);
   const T rol = L[0], vnl = L[1], vtl = L[2], vul = L[3], btl = L[4], bul = L[5], prl = L[6];
   const T ror = R[0], vnr = R[1], vtr = R[2], vur = R[3], btr = R[4], bur = R[5], prr = R[6];
@@ -891,14 +894,14 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   T dvtl = T(0.0), dvul = T(0.0), dbtl = T(0.0), dbul = T(0.0);
   T dvtr = T(0.0), dvur = T(0.0), dbtr = T(0.0), dbur = T(0.0);
   if (dabs(rhdl) > FL_EPS) {
-    const T q = O::ratio(vnc - vnl, rhdl);
+    const T q = V::ratio(vnc - vnl, rhdl);
     dvtl = -bnc * btl * q;
     dvul = -bnc * bul * q;
     dbtl = bnc2 * btl * q * slvci;
     dbul = bnc2 * bul * q * slvci;
   }
   if (dabs(rhdr) > FL_EPS) {
-    const T q = O::ratio(vnc - vnr, rhdr);
+    const T q = V::ratio(vnc - vnr, rhdr);
     dvtr = -bnc * btr * q;
     dvur = -bnc * bur * q;
     dbtr = bnc2 * btr * q * srvci;
@@ -947,9 +950,9 @@ QAS_HD void flux_mlau(const T* L, const T* R, T bnc, T gamma, T dv0, T dv1, T* F
   rv2b2 *= rv2b2;
   T vb3 = T(0.0);
   if (rv2b2 > FL_EPS * FL_EPS) {
-    // (in FP32 a denominator of eight factors may leave the reciprocal's range)
-    using V = typename std::conditional<std::is_same<T, float>::value, PlainOps, O>::type;
-    vb3 = V::ratio(+(fmt * vnc + fbt * bnc) * (fmt * bnc + fbt * mflux) +
+    // (operators: products of many factors; in FP32 the denominator may leave
+    // the reciprocal's range, in FP64 the numerator that of quot)
+    vb3 = PlainOps::ratio(+(fmt * vnc + fbt * bnc) * (fmt * bnc + fbt * mflux) +
                     (fmu * vnc + fbu * bnc) * (fmu * bnc + fbu * mflux),
                 rv2b2);
   }
@@ -1003,10 +1006,10 @@ QAS_HD void flux_roe(const T* L, const T* R, T bnc, T gamma, T* F)
   const T ca2 = bnbar * bnbar * robari;
   const T cb2 = (btbar * btbar + bubar * bubar) * robari;
   const T cf2 = T(0.5) * (a2 + O::root(cb2 * (a2 + c2 + ca2) + (c2 - ca2) * (c2 - ca2)));
-  const T cs2 = O::ratio(c2 * ca2, cf2);
+  const T cs2 = c2 * ca2 / cf2;  // (operators: the normal field may be of any size)
   const T cf = O::root(cf2);
-  const T cs = O::root(cs2);
-  const T ca = O::root(ca2);
+  const T cs = dsqrt(cs2);
+  const T ca = dsqrt(ca2);
   const T c = O::root(c2);
   const T cfi = O::inv(cf);
   const T sgr1 = btbar * btbar + bubar * bubar - FL_EPS;
@@ -1186,14 +1189,14 @@ QAS_HD T cuct_weight(T ro0, T ro1, T ro2, T ro3, T va0, T va1, T va2, T va3, T v
 {
   const T eps = T(1e-12);
   T roc = T(0.25) * (ro0 + ro1 + ro2 + ro3);
-  roc = FastOps::inv(FastOps::root(roc));
+  roc = T(1.0) / dsqrt(roc);
   T vac = T(0.25) * (va0 + va1 + va2 + va3);
   T vbc = T(0.25) * (vb0 + vb1 + vb2 + vb3);
   const T bac = T(0.5) * (ba1 + ba3);
   const T bbc = T(0.5) * (bb2 + bb3);
   vac = dabs(vac) + dabs(bac * roc);
   vbc = dabs(vbc) + dabs(bbc * roc);
-  return FastOps::ratio(vac + T(0.5) * eps, vac + vbc + eps);
+  return (vac + T(0.5) * eps) / (vac + vbc + eps);
 }
 
 // rk_updt (common/common_func.h:28-32)

@@ -156,3 +156,23 @@ def test_flux_across_magnitudes(pts, oracle, rmn):
     q[:, 3 * k:4 * k, 1] = bn[3 * k:4 * k] / np.sqrt(q[0, 3 * k:4 * k, 0]) * rng.choice([-1.0, 1.0], k)
     out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
     assert _eq_nan(out, ref)
+
+
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+def test_flux_with_tiny_velocities_and_fields(pts, oracle, rmn):
+    """Densities and pressures of order 1 with some velocities and field
+    components from 1e-320 to 1e-50, as in the tails of a localised
+    perturbation: their squares, the normal field's above all, are denormal or
+    underflow.  The oracle's values."""
+    print("case: flux, tiny velocities and fields, rmn", rmn, flush=True)
+    rng = np.random.default_rng(50 + rmn)
+    n = 40000
+    for lo, hi in ((-100, -50), (-165, -140), (-200, -100), (-290, -200), (-320, -290)):
+        q = rng.uniform(0.5, 2.0, (2, n, 7)) * np.where(np.arange(7) % 6 == 0, 1.0, rng.choice([-1.0, 1.0], (2, n, 7)))
+        bn = rng.uniform(-2.0, 2.0, n)
+        dv = rng.uniform(-0.2, 0.2, (n, 2))
+        q[1, : n // 4] = q[0, : n // 4]  # equal sides but for what is tiny
+        for a in (q[..., 1], q[..., 2], q[..., 3], q[..., 4], q[..., 5], bn):
+            a *= np.where(rng.random(n) < 0.7, 10.0 ** rng.uniform(lo, hi, a.shape), 1.0)
+        out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
+        assert _eq_nan(out, ref), (lo, hi)
