@@ -176,3 +176,22 @@ def test_flux_with_tiny_velocities_and_fields(pts, oracle, rmn):
             a *= np.where(rng.random(n) < 0.7, 10.0 ** rng.uniform(lo, hi, a.shape), 1.0)
         out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
         assert _eq_nan(out, ref), (lo, hi)
+
+
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+@pytest.mark.parametrize("side", ["left", "right", "both"])
+@pytest.mark.parametrize("var", [0, 6])
+def test_flux_of_broken_states(pts, oracle, rmn, side, var):
+    """A negative density or pressure on either side: the oracle's values, NaN
+    where it has NaN (a run that breaks down must show it)."""
+    print("case: flux, negative variable", var, side, "rmn", rmn, flush=True)
+    rng = np.random.default_rng(60 + rmn)
+    n = 20000
+    q = rng.uniform(0.5, 2.0, (2, n, 7)) * np.where(np.arange(7) % 6 == 0, 1.0, rng.choice([-1.0, 1.0], (2, n, 7)))
+    bn = rng.uniform(-2.0, 2.0, n)
+    bn[: n // 8] = 0.0
+    dv = rng.uniform(-0.2, 0.2, (n, 2))
+    for s in {"left": (0,), "right": (1,), "both": (0, 1)}[side]:
+        q[s, :, var] *= -1.0
+    out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
+    assert _eq_nan(out, ref)
