@@ -62,12 +62,14 @@ constexpr int YRP = 72;        // LDS column length: 4 columns x 8 rows fall on 
 // sweeps built with FMA contraction (qas_fma64.hip) are the same template
 // under FMA = 1, so their kernel symbols differ from the bit-exact ones.
 // Registers: FP64 keeps the stencil in registers (HLLD 146 VGPRs, 3 waves per
-// SIMD), except the batch's HLLD instance, whose characteristic fields read it
-// from LDS again (126 VGPRs, 4 waves per SIMD: 24 domains 228 -> 220 us a
-// launch; one 64^2 domain, a single round of wavefronts, took 11.5 us that way
-// against 10.6).  FP32 tiles hold FP32 values, read from LDS (113 VGPRs).
+// SIMD), except the batch's HLLD instance of ODR 4, whose characteristic fields
+// read it from LDS again (126 VGPRs, 4 waves per SIMD: 24 domains 228 -> 220 us
+// a launch; one 64^2 domain, a single round of wavefronts, took 11.5 us that
+// way against 10.6).  At ODR 3 that form spills 76 bytes per lane (24 domains
+// 256 us, in registers 210); at ODR 1 and 2 the two take the same time.  FP32
+// tiles hold FP32 values, read from LDS (113 VGPRs).
 template <int RMN, int ODR, typename T, bool BATCH, bool GRAV = false, int FMA = 0>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH && RMN == 1 ? 4 : 3)) void k_sweep2d_y(
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH && RMN == 1 && ODR == 4 ? 4 : 3)) void k_sweep2d_y(
     StagePtrs p_arg, Geo g_arg, BcFlags bc_arg, double gam, int bundle_arg, const BatchInst* I, const int* off,
     int ninst, int stage)
 {
@@ -149,7 +151,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH &
   const int rb = lane + 2;  // this lane's cell in the tile
   // the stencil in registers, or left in LDS for each characteristic field to
   // read its part
-  constexpr bool IN_LDS = sizeof(T) == 4 || (BATCH && RMN == 1);
+  constexpr bool IN_LDS = sizeof(T) == 4 || (BATCH && RMN == 1 && ODR == 4);
   const LdsStencil<T, T, YC * YRP, 1> sl{&sh[0][w][rb]};
   T sr[7][5];
   if constexpr (!IN_LDS) {
@@ -264,7 +266,9 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN >= 2 ? 3 : 4) : (BATCH &
 // each characteristic field reads its part again: 116 VGPRs and 35 fewer loads
 // a lane, MLAU at 2048^2 247 -> 202 us.  FP64 loads its stencil straight into
 // registers: from LDS it gained nothing (142 VGPRs as before, 83.3 us against
-// 82.2 at 1024^2; held to 4 waves per SIMD it spilled, 105 us).
+// 82.2 at 1024^2; held to 4 waves per SIMD it spilled, 105 us).  3 waves per
+// SIMD for every FP64 instance: Roe and MLAU with gravity at ODR 4 spill 20
+// bytes per lane for it, 512 x 1024 50.5 us against 53.4 in 2 waves without.
 // LDS per lane: the cell's 7 values (then its 6 fluxes) and, apart from them,
 // 8 face values and the sensor; odd strides, so that 64 lanes fall on different banks.
 constexpr int XS = 7, XL = 9;

@@ -107,6 +107,11 @@ __device__ __forceinline__ Prim3d prim3d_cell(const StagePtrs& p, const Geo& g, 
 // direct per-lane sweep.  z and y sweeps at 128^3 (FP64) 302 and 228 us with
 // runs cut by column and shuffles, 257 and 196 this way; at 200^3 (mixed, the
 // tile in FP32) 602 and 447 -> 562 and 329.
+// Column length of the results in LDS: 64 are used; 70, with the tile's 72, lets
+// four FP64 workgroups into a CU's 160 KB (at 72 three: 128^3 HLLD ODR 1 y 139.6 us
+// against 129.9, ODR 3 184 against 170; at 64 the write-back's 4 columns fall
+// on the same banks, Roe 1 to 2 % slower).
+constexpr int YO3 = 70;
 template <int DIR, int RMN, int ODR, typename T>
 __device__ __forceinline__ void sweep3d_t(const StagePtrs& p, const Geo& g, const BcFlags& bc, double gam, int bundle)
 {
@@ -115,7 +120,7 @@ __device__ __forceinline__ void sweep3d_t(const StagePtrs& p, const Geo& g, cons
   constexpr int TB = (DIR + 2) % 3;
   constexpr int LB = DIR == 2 ? 1 : 2;  // the other transverse axis (x is the column axis)
   __shared__ T sh[9][YC][YRP];      // ro vn vt vu bt bu pr cn bf
-  __shared__ T so[9][YC][YRP];      // 5 fluxes, 4 face parts
+  __shared__ T so[9][YC][YO3];      // 5 fluxes, 4 face parts
   const int dims[3] = {g.nx, g.ny, g.nz};
   const long long strd[3] = {1, g.sy, g.sz};
   const int ncg = (g.nx + YC - 1) / YC;
@@ -293,8 +298,10 @@ __global__ __launch_bounds__(256, 2) void k_sweep3d_t(StagePtrs p, Geo g, BcFlag
 // Runs of the domain's cells in memory order, states and fluxes handed over
 // through LDS as in the 2D x sweep; it runs after the z and y sweeps and
 // applies the RK stage sum.  128^3 (FP64) 272 -> 186 us, 200^3 (mixed) 448 -> 386.
+// Waves per SIMD: FP32 MLAU below ODR 4 needs 5 (128^3, ODR 3 113 us against 126;
+// ODR 4 takes 121 VGPRs).
 template <int RMN, int ODR, typename T, int FMA = 0>
-__global__ __launch_bounds__(256, sizeof(T) == 4 ? 4 : (RMN == 1 ? 3 : 2)) void k_sweep3d(StagePtrs p, Geo g, BcFlags bc, double gam, int)
+__global__ __launch_bounds__(256, sizeof(T) == 4 ? (RMN == 3 && ODR < 4 ? 5 : 4) : (RMN == 1 ? 3 : 2)) void k_sweep3d(StagePtrs p, Geo g, BcFlags bc, double gam, int)
 {
   extern __shared__ double x_lds[];
   constexpr int XL3 = 11;  // 7 states, 2 B-flux states, the sensor; odd
