@@ -150,6 +150,140 @@ __global__ __launch_bounds__(256) void k_emf3d(StagePtrs p, Geo g, int ctw, int 
   }
 }
 
+// Large domains: all three components of the edges of a column in one thread,
+// marching along z; the four z-interpolated face-part arrays sit in register
+// windows and the cells of the plane behind are carried.  ro, v and B are read
+// once for the three, where k_emf3d's Ez blocks, which run after the others,
+// read them again; at 256 VGPRs (2 wavefronts per SIMD) and 32 planes a thread
+// it needs many columns.  The line lies where a face-part array no longer stays
+// in the caches: k_emf3d and this form take 279 and 292 us at 160^3 FP64 (38
+// MB an array), 544 and 485 at 200^3 (72 MB), 8.92 and 6.47 ms at 512^3; mixed
+// 338 and 348 us at 200^3 (36 MB), 368 and 361 at 64^2 x 2048 (43 MB), 507 and
+// 472 at 224^3 (50 MB), 838 and 834 at 512^2 x 64 (78 MB), 5.43 and 4.51 ms at
+// 512^3.  (In tiles of 64 x 4 columns, partly empty, it took 7.27 and 4.89 ms.)
+constexpr long long EMF_ALL_MIN = 45000000;  // bytes of a face-part array
+// Interpolate the face parts (upwind fu, central fc) of a
+// sweep along axis o to the edge and combine with weight w:
+//   sgn * ((uL + uR) + w (cL + cR))
+template <int ODR, typename FT>
+__device__ __forceinline__ double emf_part(const double* fu, const double* fc, long long ss, long long o, double w,
+                                           double sgn)
+{
+  double a[5], b[5], ul0, ur0, ul1, ur1, dum;
+#pragma unroll
+  for (int m = 0; m < 5; m++) { a[m] = load_as<FT>(fu, ss + (m - 3) * o); b[m] = load_as<FT>(fc, ss + (m - 3) * o); }
+  lin5<ODR>(a, ul0, dum);
+  lin5<ODR>(b, ul1, dum);
+#pragma unroll
+  for (int m = 0; m < 5; m++) { a[m] = load_as<FT>(fu, ss + (m - 2) * o); b[m] = load_as<FT>(fc, ss + (m - 2) * o); }
+  lin5<ODR>(a, dum, ur0);
+  lin5<ODR>(b, dum, ur1);
+  return sgn * ((ul0 + ur0) + w * (ul1 + ur1));
+}
+
+constexpr int EMF_KC = 32;  // planes per thread
+
+template <int ODR, typename FT>
+__global__ __launch_bounds__(256) void k_emf3d_z(StagePtrs p, Geo g, int ctw, int nbxy)
+{
+  const unsigned ni = (unsigned)g.nx - 5;  // edges on [3, n-3]
+  const int L = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const int chunk = L / nbxy;
+  const unsigned q = (unsigned)(L - chunk * nbxy) * 256u + threadIdx.x;
+  const unsigned row = q / ni;
+  if (row >= (unsigned)g.ny - 5) return;  // no barriers below
+  const int i = 3 + (int)(q - row * ni), j = 3 + (int)row;
+  const int k0 = 3 + chunk * EMF_KC;
+  const int k1 = k0 + EMF_KC < g.nz - 2 ? k0 + EMF_KC : g.nz - 2;
+  const long long sy = g.sy, sz = g.sz;
+  const double* ro = p.in[0];
+  const double *bx = p.in[4], *by = p.in[5], *bz = p.in[6];
+  // z windows at planes k-3 .. k+2
+  double u2[6], c2[6], u4[6], c4[6];
+  {
+    const long long s0 = sz * k0 + sy * j + i;
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+      const long long a = s0 + (m - 3) * sz;
+      u2[m] = load_as<FT>(p.emf[2], a);
+      c2[m] = load_as<FT>(p.emf[3], a);
+      u4[m] = load_as<FT>(p.emf[4], a);
+      c4[m] = load_as<FT>(p.emf[5], a);
+    }
+  }
+  // plane k0-1 cell values used by the Ex / Ey weights
+  double ro_p = 0, ro_pi = 0, ro_pj = 0, vx_p = 0, vx_pi = 0, vy_p = 0, vy_pj = 0, vz_p = 0, vz_pi = 0, vz_pj = 0,
+         bx_p = 0, by_p = 0;
+  if (ctw) {
+    const long long s = sz * (k0 - 1) + sy * j + i;
+    ro_p = ro[s]; ro_pi = ro[s - 1]; ro_pj = ro[s - sy];
+    vx_p = load_as<FT>(p.vx, s); vx_pi = load_as<FT>(p.vx, s - 1);
+    vy_p = load_as<FT>(p.vy, s); vy_pj = load_as<FT>(p.vy, s - sy);
+    vz_p = load_as<FT>(p.vz, s); vz_pi = load_as<FT>(p.vz, s - 1); vz_pj = load_as<FT>(p.vz, s - sy);
+    bx_p = bx[s]; by_p = by[s];
+  }
+  for (int k = k0; k < k1; k++) {
+    const long long ss = sz * k + sy * j + i;
+    {
+      const long long a = ss + 2 * sz;
+      u2[5] = load_as<FT>(p.emf[2], a);
+      c2[5] = load_as<FT>(p.emf[3], a);
+      u4[5] = load_as<FT>(p.emf[4], a);
+      c4[5] = load_as<FT>(p.emf[5], a);
+    }
+    double ctz = 0.5, ctx = 0.5, cty = 0.5;
+    double ro0 = 0, roi = 0, roj = 0, vx0 = 0, vxi = 0, vy0 = 0, vyj = 0, vz0 = 0, vzi = 0, vzj = 0, bx0 = 0,
+           by0 = 0;
+    if (ctw) {
+      ro0 = ro[ss]; roi = ro[ss - 1]; roj = ro[ss - sy];
+      const double roij = ro[ss - 1 - sy];
+      vx0 = load_as<FT>(p.vx, ss); vxi = load_as<FT>(p.vx, ss - 1);
+      const double vxj = load_as<FT>(p.vx, ss - sy), vxij = load_as<FT>(p.vx, ss - 1 - sy);
+      vy0 = load_as<FT>(p.vy, ss); vyj = load_as<FT>(p.vy, ss - sy);
+      const double vyi = load_as<FT>(p.vy, ss - 1), vyij = load_as<FT>(p.vy, ss - 1 - sy);
+      vz0 = load_as<FT>(p.vz, ss); vzi = load_as<FT>(p.vz, ss - 1); vzj = load_as<FT>(p.vz, ss - sy);
+      bx0 = bx[ss]; by0 = by[ss];
+      // x-y plane for Ez: strides (1, ny)
+      ctz = cuct_weight(roij, roj, roi, ro0, vxij, vxj, vxi, vx0, vyij, vyj, vyi, vy0, bx[ss - sy], bx0, by[ss - 1],
+                        by0);
+      // y-z plane for Ex: strides (sy, sz)
+      ctx = cuct_weight(ro_pj, ro_p, roj, ro0, vy_pj, vy_p, vyj, vy0, vz_pj, vz_p, vzj, vz0, by_p, by0, bz[ss - sy],
+                        bz[ss]);
+      // z-x plane for Ey: strides (sz, 1)
+      cty = cuct_weight(ro_pi, roi, ro_p, ro0, vz_pi, vzi, vz_p, vz0, vx_pi, vxi, vx_p, vx0, bz[ss - 1], bz[ss], bx_p,
+                        bx0);
+    }
+    // Ez: x sweep B_y (t) along y, then y sweep B_x (u) along x
+    double ez = 0.0;
+    ez += emf_part<ODR, FT>(p.emf[0], p.emf[1], ss, sy, 1.0 - ctz, -0.5);
+    ez += emf_part<ODR, FT>(p.emf[6], p.emf[7], ss, 1, ctz, +0.5);
+    // Ey: x sweep B_z (u) along z, then z sweep B_x (t) along x
+    double ey = 0.0;
+    ey += emf_part_w<ODR>(u2, c2, cty, +0.5);
+    ey += emf_part<ODR, FT>(p.emf[8], p.emf[9], ss, 1, 1.0 - cty, -0.5);
+    // Ex: y sweep B_z (t) along z, then z sweep B_y (u) along y
+    double ex = 0.0;
+    ex += emf_part_w<ODR>(u4, c4, 1.0 - ctx, -0.5);
+    ex += emf_part<ODR, FT>(p.emf[10], p.emf[11], ss, sy, ctx, +0.5);
+    store_as<FT>(p.ex, ss, ex);
+    store_as<FT>(p.ey, ss, ey);
+    store_as<FT>(p.ez, ss, ez);
+    // next plane: shift the windows, carry this plane's values
+#pragma unroll
+    for (int m = 0; m < 5; m++) {
+      u2[m] = u2[m + 1];
+      c2[m] = c2[m + 1];
+      u4[m] = u4[m + 1];
+      c4[m] = c4[m + 1];
+    }
+    ro_p = ro0; ro_pi = roi; ro_pj = roj;
+    vx_p = vx0; vx_pi = vxi;
+    vy_p = vy0; vy_pj = vyj;
+    vz_p = vz0; vz_pi = vzi; vz_pj = vzj;
+    bx_p = bx0; by_p = by0;
+  }
+}
+
 // ------------------------------------------------------------------ CT
 // Staggered-B update (mhd_updt3d_ctb, common/mhd_func.c:302-325), marching
 // along z: one thread per (i, j) column of the x-y plane over kc planes.  The
@@ -278,9 +412,13 @@ hipError_t launch_stage3d(qas_ctx* c, const StagePtrs& p)
   const int cxy = (int)nblk3((long long)(g.nx - 7) * (g.ny - 7), 256);
   const int ck = march_chunk(cxy, g.nz - 7, 8192);
   const unsigned nct = (unsigned)(cxy * (int)nblk3(g.nz - 7, ck));
+  const unsigned nemfz = (unsigned)(exy * (int)nblk3(g.nz - 5, EMF_KC));
+  const bool all = g.nd * (f32 ? 4 : 8) >= EMF_ALL_MIN;
   // (the face parts and edges are stored in the sweep precision)
 #define QAS_EMF_CT(O)                                                                                             \
-  if (f32) QAS_LAUNCH(c, QAS_K_EMF, (k_emf3d<O, float>), nemf, 256, 0, st, p, g, c->s.ctw, exy, exz, nexy, ek);   \
+  if (all && f32) QAS_LAUNCH(c, QAS_K_EMF, (k_emf3d_z<O, float>), nemfz, 256, 0, st, p, g, c->s.ctw, exy);             \
+  else if (all) QAS_LAUNCH(c, QAS_K_EMF, (k_emf3d_z<O, double>), nemfz, 256, 0, st, p, g, c->s.ctw, exy);              \
+  else if (f32) QAS_LAUNCH(c, QAS_K_EMF, (k_emf3d<O, float>), nemf, 256, 0, st, p, g, c->s.ctw, exy, exz, nexy, ek);   \
   else QAS_LAUNCH(c, QAS_K_EMF, (k_emf3d<O, double>), nemf, 256, 0, st, p, g, c->s.ctw, exy, exz, nexy, ek);      \
   if (f32) QAS_LAUNCH(c, QAS_K_CT, (k_ct3d<O, float>), nct, 256, 0, st, p, g, cxy, ck);                           \
   else QAS_LAUNCH(c, QAS_K_CT, (k_ct3d<O, double>), nct, 256, 0, st, p, g, cxy, ck);

@@ -180,6 +180,41 @@ def test_3d_runs_chunks_and_ghosts_vs_oracle(qas, oracle, nx, ny, nz, rmn, odr, 
     assert np.array_equal(out, ref)
 
 
+@pytest.mark.parametrize("rmn,odr,ctw,precision", [(1, 4, 1, 0), (1, 4, 0, 0), (3, 3, 1, 0), (0, 2, 1, 0), (2, 1, 1, 0),
+                                                   (1, 4, 1, 1), (3, 3, 0, 1)])
+def test_3d_large_domain_is_its_tiles(qas, oracle, rmn, odr, ctw, precision):
+    """Above 45 MB a face-part array the edge EMFs come from the form with all
+    three components in a thread.  A periodic domain laid side by side is
+    periodic with the same period, cell for cell: the large domain's step must
+    be the small one's (other EMF form; in FP64 the oracle's) repeated."""
+    n, rep = (20, 28, 24), (9, 7, 8) if precision == 0 else (12, 7, 9)  # nz, ny, nx; partly empty last chunk
+    rng = np.random.default_rng(5)
+    shape = tuple(m + 8 for m in n)
+    z, y, x = np.meshgrid(*[2 * np.pi * (np.arange(m) - 4) / (m - 8) for m in shape], indexing="ij")
+    f = [sum(rng.uniform(0.2, 0.5) * np.cos(a * x + b * y + c * z + rng.uniform(0, 6)) for a, b, c in
+             ((1, 0, 1), (0, 1, 1), (1, 1, 0))) for _ in range(8)]
+    st = np.stack([1.5 + 0.3 * f[0], f[1], f[2], f[3], f[4], f[5], f[6], 8.0 + f[7]])
+    inner = st[:, 4:-4, 4:-4, 4:-4]
+    big = np.tile(inner, (1,) + rep)
+    big = np.pad(big, ((0, 0),) + ((4, 4),) * 3, mode="wrap")
+    st = np.pad(inner, ((0, 0),) + ((4, 4),) * 3, mode="wrap")
+    assert big[0].size * (4 if precision else 8) >= 45000000 > st[0].size * 8
+    _say("3d large domain is its tiles", rmn, odr, ctw, precision, big.shape)
+    out = []
+    for u in (st, big):
+        with qas.Solver(u.shape[1:], 0.1, 0.12, 0.11, rmn=rmn, odr=odr, ctw=ctw, precision=precision) as s:
+            s.upload(u)
+            s.run(1, flg=0, dt=2e-3, history=False)
+            out.append(s.download())
+    if precision == 0:
+        cfg = oracle.make_cfg(st.shape[1:], 0.1, 0.12, 0.11, rmn=rmn, odr=odr, ctw=ctw)
+        ref = st.copy()
+        oracle.run(cfg, ref, 1, 0, dt=2e-3)
+        assert np.array_equal(out[0], ref)
+    want = np.pad(np.tile(out[0][:, 4:-4, 4:-4, 4:-4], (1,) + rep), ((0, 0),) + ((4, 4),) * 3, mode="wrap")
+    assert np.isfinite(out[0]).all() and np.array_equal(out[1], want)
+
+
 @pytest.mark.parametrize("n", [8, 52, 53, 57, 112, 4097])
 @pytest.mark.parametrize("dn", [0, 1, -1, 2, -2])
 def test_1d_stage_and_ghosts_vs_oracle(qas, oracle, n, dn):
