@@ -122,10 +122,13 @@ int qas_use_graphs(qas_ctx *c, int on);
 /* 2D launch shape (no counterpart in the reference: its loops have no
  * launch geometry): x-sweep wavefronts per workgroup (xwpb 1, 2, 4) and the
  * workgroup size of the element-wise kernels (ewb 64, 128, 256).  Every
- * shape gives the same results.  qas_tune times RK stage 1 of the uploaded
+ * shape gives the same results.  qas_tune times the RK stages of the uploaded
  * state in each of the 9 shapes and keeps the fastest (the state is not
  * changed); the first qas_run of a 2D context calls it unless a shape was
- * set.  qas_set_shape fixes a shape, qas_shape reports the current one
+ * set.  Domains of up to 300 x 300 cells, ghosts included, have no
+ * element-wise launch in a stage: ewb has no effect there and qas_tune times
+ * the three xwpb at ewb 256.  qas_set_shape fixes a shape, qas_shape reports the
+ * current one
  * (default 4, 256).  1D and 3D have one shape. */
 int qas_tune(qas_ctx *c);
 int qas_set_shape(qas_ctx *c, int xwpb, int ewb);

@@ -389,8 +389,10 @@ int qas::ctx_tune(qas_ctx* c)
   c->tuned = true;
   if (c->g.ndim != 2) return QAS_OK;  // one shape in 1D and 3D
   const int cand[9][2] = {{4, 256}, {2, 256}, {1, 256}, {4, 128}, {2, 128}, {1, 128}, {4, 64}, {2, 64}, {1, 64}};
+  // (no element-wise launch in the stages of a small domain: its three shapes)
+  const int nshape = fused_emf_ct(c->geo) ? 3 : 9;
   const int A = c->cur, B = (c->cur + 1) % 3;
-  constexpr int NSHAPE = 9, NREP = 3, NROUND = 2;
+  constexpr int NREP = 3, NROUND = 2;
   const int R = c->s.r_k;
   const int C = (c->cur + 2) % 3;
   // stage rk reads s_in[rk] and writes s_out[rk] (R_K 1: A -> B; 2: A -> B -> C;
@@ -401,10 +403,10 @@ int qas::ctx_tune(qas_ctx* c)
   hipEvent_t e0 = nullptr, e1 = nullptr;
   QAS_CHECK(c, hipEventCreate(&e0));
   hipError_t e = hipEventCreate(&e1);
-  float tmin[NSHAPE];
-  for (int k = 0; k < NSHAPE; k++) tmin[k] = -1.0f;
+  float tmin[9];
+  for (int k = 0; k < nshape; k++) tmin[k] = -1.0f;
   for (int round = -1; round < NROUND && e == hipSuccess; round++) {  // round -1: warm-up
-    for (int k = 0; k < NSHAPE && e == hipSuccess; k++) {
+    for (int k = 0; k < nshape && e == hipSuccess; k++) {
       c->xwpb = cand[k][0];
       c->ewb = cand[k][1];
       e = hipEventRecord(e0, c->stream);
@@ -420,7 +422,7 @@ int qas::ctx_tune(qas_ctx* c)
     }
   }
   int bi = 0;
-  for (int k = 1; k < NSHAPE; k++)
+  for (int k = 1; k < nshape; k++)
     if (tmin[k] >= 0.0f && tmin[k] < tmin[bi]) bi = k;
   (void)hipEventDestroy(e0);
   if (e1) (void)hipEventDestroy(e1);

@@ -326,6 +326,10 @@ inline bool prof_slot(qas_ctx* c, int kid, hipEvent_t* e0, hipEvent_t* e1)
 
 // ---- launchers (defined in the per-dimension translation units) ----
 namespace qas {
+// 2D domains whose corner EMF, CT and ghost fill are one launch (k_emfct2d,
+// which says why): cells with ghosts
+constexpr long long FUSE_MAX = 300LL * 300;
+inline bool fused_emf_ct(const Geo& g) { return g.ndim == 2 && g.nd <= FUSE_MAX; }
 hipError_t launch_bound(qas_ctx* c, double* const f[8], int nvar);
 hipError_t launch_cfl(qas_ctx* c, const double* const U[8]);
 hipError_t launch_cfl_finalize(qas_ctx* c, double* hist_slot);

@@ -64,7 +64,6 @@ __global__ __launch_bounds__(256) void k_ctb2d(StagePtrs p, Geo g, BcFlags bc, c
 // 64^2, 8.6 against 4.6 + 4.8 at 256^2, 12.8 against 5.3 + 6.2 at 517 x 389,
 // 45 against 19 + 16 at 1024^2.  Never stored: nothing else reads them.
 constexpr int FT_X = 32, FT_Y = 8, FT_NB = 448;
-constexpr long long FUSE_MAX = 300LL * 300;
 template <int ODR, typename FT>
 __global__ __launch_bounds__(FT_NB) void k_emfct2d(StagePtrs p, Geo g, BcFlags bc, int ctw, const double* phi,
                                                   double gfac, long long nghost, int ntx, int nbct)
@@ -134,7 +133,7 @@ hipError_t launch_stage2d(qas_ctx* c, const StagePtrs& p, bool faces_only)
   const int eb = c->ewb;
   const unsigned nbct = nblk(nc, eb);
 
-  const bool fuse = (long long)g.nx * g.ny <= FUSE_MAX;
+  const bool fuse = fused_emf_ct(g);
   const int ntx = (g.nx - 7 + FT_X - 1) / FT_X, nbt = ntx * ((g.ny - 7 + FT_Y - 1) / FT_Y);
 #define QAS_FUSED(O)                                                                                       \
   if (f32) QAS_LAUNCH(c, QAS_K_CT, (k_emfct2d<O, float>), nbt + nblk(nghost * 8, FT_NB), FT_NB, 0, st, p, g, c->bc, \

@@ -512,6 +512,32 @@ def test_launch_shapes_bit_identical(qas, oracle):
         assert np.array_equal(h, href)
 
 
+@pytest.mark.parametrize("nx,ny", [(292, 292), (320, 300)])
+def test_launch_shapes_where_they_matter(qas, oracle, nx, ny):
+    """The largest domain whose corner EMF and CT are one launch (its tuned
+    shape has the default element-wise size, which no launch of it uses), and
+    one with separate launches, whose workgroup size is ewb: the oracle's bits
+    in every shape."""
+    from qasmhd_amd import problems
+    p = problems.turbulence2d(n=nx, ny=ny, seed=6)
+    _say("launch shapes", nx, ny)
+    cfg = oracle.make_cfg(p.state.shape[1:], p.dx, p.dy, gam=p.gam)
+    ref = p.state.copy()
+    href, _ = oracle.run(cfg, ref, 2, 1)
+    for xwpb, ewb in ((1, 64), (2, 128), (4, 256), (1, 256), (4, 64)):
+        with qas.solver_for(p) as s:
+            s.set_shape(xwpb, ewb)
+            s.upload(p.state)
+            h, _ = s.run(2, flg=1)
+            assert s.shape_now() == (xwpb, ewb)
+            assert np.array_equal(s.download(), ref) and np.array_equal(h, href), (xwpb, ewb)
+    for _ in range(8):
+        with qas.solver_for(p) as s:
+            s.upload(p.state)
+            xwpb, ewb = s.tune()
+            assert xwpb in (1, 2, 4) and (ewb == 256 if (nx + 8) * (ny + 8) <= 300 * 300 else ewb in (64, 128, 256))
+
+
 @pytest.mark.parametrize("nsteps", [7, 10])
 def test_graph_replay_matches_direct_launches(qas, oracle, nsteps):
     """qas_run with captured 2-step graphs == host-launched steps == oracle,
