@@ -55,15 +55,18 @@ __global__ __launch_bounds__(256) void k_ctb2d(StagePtrs p, Geo g, BcFlags bc, c
     ctb2d_at<ODR>(p, g, bc, phi, gfac, nghost, (long long)(b - nbct) * blockDim.x + threadIdx.x, false);
 }
 
-// Small domains: corner EMF, CT and the ghost fill in one launch.  A workgroup
-// forms the corner EMFs of a 32 x 8 tile of faces (35 x 11 corners, one per
-// thread of its 448) in LDS and updates the faces from there; the last blocks
-// fill the cell-centred ghosts.  The corners of a tile's rim are formed by its
+// Small domains (fused_emf_ct): corner EMF, CT and the ghost fill in one launch.
+// A workgroup forms the corner EMFs of a 32 x 8 tile of faces (35 x 11 corners,
+// one per thread) in LDS and updates the faces from there; the last blocks fill
+// the cell-centred ghosts.  The corners of a tile's rim are formed by its
 // neighbours too (1.5 per face), which costs more than the second launch once
-// a launch fills the chip: 7.3 us against 4.0 + 4.8 and a gap of about 1 at
-// 64^2, 8.6 against 4.6 + 4.8 at 256^2, 12.8 against 5.3 + 6.2 at 517 x 389,
-// 45 against 19 + 16 at 1024^2.  Never stored: nothing else reads them.
-constexpr int FT_X = 32, FT_Y = 8, FT_NB = 448;
+// a launch fills the chip.  A whole stage, fused against separate (FP64, ODR 4):
+// 26.3 against 28.0 us at 64^2, 37.4 against 37.8 at 292^2, 43.3 against 43.7
+// at 350^2, 46.7 against 46.0 at 400^2, 57.7 against 56.3 at 450^2.  Never
+// stored: nothing else reads them.  512 threads, though 385 have a corner: after
+// workgroups of 448, an odd number of wavefronts, the next stage's x sweep
+// (2 wavefronts a workgroup) took 15.1 us at 256^2 instead of 12.4.
+constexpr int FT_X = 32, FT_Y = 8, FT_NB = 512;
 template <int ODR, typename FT>
 __global__ __launch_bounds__(FT_NB) void k_emfct2d(StagePtrs p, Geo g, BcFlags bc, int ctw, const double* phi,
                                                   double gfac, long long nghost, int ntx, int nbct)
