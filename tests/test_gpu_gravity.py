@@ -36,6 +36,26 @@ def test_gravity_run_vs_oracle(oracle, rmn, odr, r_k, flg):
     assert np.array_equal(out, ref)
 
 
+@pytest.mark.parametrize("rmn,odr", [(2, 4), (1, 2), (0, 4), (3, 3)])
+def test_gravity_with_separate_ct_launch_vs_oracle(oracle, rmn, odr):
+    """Above 300^2 cells the CT and the ghost fill, with the hydrostatic energy
+    ghosts, are a launch of their own (the smaller cases' are fused with the
+    corner EMF)."""
+    from qasmhd_amd import capi, problems
+    _say("case: gravity, separate CT launch, RTI 96x1024, rmn", rmn, "odr", odr)
+    p, phi = problems.rayleigh_taylor2d(nx=96, ny=1024, dv=0.05)
+    cfg = oracle.make_cfg(p.state.shape[1:], p.dx, p.dy, gam=p.gam, rmn=rmn, odr=odr, dn=p.dn, phi=phi)
+    ref = p.state.copy()
+    h_ref, _ = oracle.run(cfg, ref, 2, 1)
+    with capi.solver_for(p, rmn=rmn, odr=odr) as s:
+        s.upload(p.state)
+        s.set_gravity(phi)
+        hist, _ = s.run(2, flg=1)
+        out = s.download()
+    assert np.isfinite(ref).all()
+    assert np.array_equal(hist, h_ref) and np.array_equal(out, ref)
+
+
 def test_gravity_steps_and_graph_replay(oracle):
     """qas_step / qas_bound / qas_cfl_dt individually and a long qas_run
     (graph replays of step pairs) against the oracle."""

@@ -176,6 +176,28 @@ def test_mixed_at_small_speeds(odr, rmn):
         assert max(e) < 1e-6
 
 
+@pytest.mark.parametrize("n,ny", [(64, 48), (320, 300), (520, 516)])
+@pytest.mark.parametrize("odr", [1, 2, 3, 4])
+def test_mixed_l1_error_by_size_and_order(odr, n, ny):
+    """The three forms of the corner EMF (fused, one and two corners a thread)
+    at every order: an FP32 rounding's error against FP64 after 4 steps."""
+    from qasmhd_amd import capi, problems
+    p = problems.turbulence2d(n=n, ny=ny, seed=3)
+    with capi.solver_for(p) as s:
+        s.upload(p.state)
+        dt = s.cfl_dt()
+    out = []
+    for precision in (0, 1):
+        with capi.solver_for(p, odr=odr, precision=precision) as s:
+            s.upload(p.state)
+            s.run(4, flg=0, dt=dt, history=False)
+            out.append(s.download())
+    I = (slice(4, -4), slice(4, -4))
+    e = [l1rel(out[1][m][I], out[0][m][I]) for m in (0, 4, 5, 7)]
+    _say("mixed vs fp64, odr %d, %d x %d: L1 of ro, bx, by, en %.2e %.2e %.2e %.2e" % (odr, n, ny, *e))
+    assert max(e) < 1e-6
+
+
 def test_mixed_l1_error_vs_oracle(oracle):
     """The mixed path's L1 error measured against the oracle itself (the
     CPU restatement of the reference) rather than through the FP64 HIP

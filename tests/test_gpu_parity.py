@@ -98,8 +98,10 @@ def test_2d_vs_oracle(qas, oracle, seed, n, ny, rmn, odr):
 def test_2d_column_emf_vs_oracle(qas, oracle, rmn, odr, walls):
     """Domains of 512^2 corners and more compute two EMF corners of a column
     per thread (k_emf2d<ODR, FT, 2>): the same arithmetic per corner as the
-    one-corner form the small cases run, for every ODR's interpolation; a
-    ragged last column (an odd corner count along y) and walls."""
+    one-corner forms (fused with the CT up to 300^2 cells, k_emf2d<ODR, FT, 1>
+    between, test_2d_separate_emf_and_ct_vs_oracle), for every ODR's
+    interpolation; a ragged last column (an odd corner count along y) and
+    walls."""
     from qasmhd_amd import problems
     p = problems.turbulence2d(n=516, ny=518, seed=7, vrms=0.8)
     dn = np.zeros((3, 8), dtype=int)
@@ -113,6 +115,31 @@ def test_2d_column_emf_vs_oracle(qas, oracle, rmn, odr, walls):
     ref = p.state.copy()
     h_ref, dt_ref = oracle.run(cfg, ref, 2, 1)
     with qas.Solver(p.state.shape[1:], p.dx, p.dy, gam=p.gam, rmn=rmn, odr=odr, dn=dn) as s:
+        s.upload(p.state)
+        hist, dt_now = s.run(2, flg=1)
+        out = s.download()
+    assert np.isfinite(ref).all()
+    assert np.array_equal(hist, h_ref) and dt_now == dt_ref
+    assert np.array_equal(out, ref)
+
+
+@pytest.mark.parametrize("rmn,odr,ctw,walls", [(1, 1, 1, False), (0, 2, 1, True), (2, 3, 0, True), (3, 4, 1, True),
+                                               (1, 3, 1, False)])
+def test_2d_separate_emf_and_ct_vs_oracle(qas, oracle, rmn, odr, ctw, walls):
+    """Between 300^2 cells and 512^2 corners the corner EMF (one corner a
+    thread) and the CT with the ghost fill are launches of their own: every
+    ODR's interpolation, walls, with and without the upwind weight."""
+    from qasmhd_amd import problems
+    p = problems.turbulence2d(n=330, ny=301, seed=8, vrms=0.8)
+    dn = np.zeros((3, 8), dtype=int)
+    if walls:
+        dn[0] = [2] * 8
+        dn[1] = [1, 1, -1, 1, 1, -1, 1, 1]
+    _say("2d separate EMF and CT vs oracle", rmn, odr, ctw, walls)
+    cfg = oracle.make_cfg(p.state.shape[1:], p.dx, p.dy, gam=p.gam, rmn=rmn, odr=odr, ctw=ctw, dn=dn)
+    ref = p.state.copy()
+    h_ref, dt_ref = oracle.run(cfg, ref, 2, 1)
+    with qas.Solver(p.state.shape[1:], p.dx, p.dy, gam=p.gam, rmn=rmn, odr=odr, ctw=ctw, dn=dn) as s:
         s.upload(p.state)
         hist, dt_now = s.run(2, flg=1)
         out = s.download()
