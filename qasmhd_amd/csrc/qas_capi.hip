@@ -67,7 +67,9 @@ static std::string validate(const qas_grid* g, const qas_scheme* s)
       if (n[a] != 1 || off[a] != 0) return "inactive axes must have n = 1 and no ghosts";
     }
   }
-  if ((long long)g->nx * g->ny * g->nz > (1LL << 40)) return "grid too large";
+  // (cells are counted in 32 bits in places; an array of 2^31 is past the
+  // memory of the device: 24 arrays and scratch of 17 GB each)
+  if ((double)g->nx * g->ny * g->nz >= 0x1p31) return "grid too large: 2^31 cells or more";
   if (s->rmn < 0 || s->rmn > 3) return "rmn must be 0..3";
   if (s->odr < 1 || s->odr > 4) return "odr must be 1..4";
   if (s->r_k < 1 || s->r_k > 3) return "r_k must be 1..3";

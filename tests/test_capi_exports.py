@@ -58,3 +58,15 @@ def test_no_fallback_without_library_or_device():
     assert r.returncode == 0, r.stderr
     assert "E1 libqasmhd_amd.so is not built" in r.stdout
     assert "E2 qas_create:" in r.stdout and "hipErrorNoDevice" in r.stdout
+
+
+@pytest.mark.parametrize("shape", [(1 << 16, 1 << 15), (1 << 15, 1 << 16), (1 << 11, 1 << 10, 1 << 10),
+                                   ((1 << 31) - 1,) * 2, ((1 << 31) - 1,) * 3])
+def test_grid_of_2_to_the_31_cells_is_refused(shape):
+    """Cells are counted in 32 bits in the ghost fill and the x sweeps: such a
+    grid is refused by the arguments' check, before any device call."""
+    from qasmhd_amd import capi
+    if not os.path.exists(capi.LIB_PATH):
+        pytest.skip("libqasmhd_amd.so not built here")
+    with pytest.raises(capi.QasError, match="grid too large"):
+        capi.Solver(shape, 1.0, 1.0, 1.0)
