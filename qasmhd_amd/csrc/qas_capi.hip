@@ -13,10 +13,6 @@
 
 #include "qas_internal.hpp"
 
-namespace qas {
-hipError_t launch_record_dt(qas_ctx* c, double* slot);
-}
-
 using namespace qas;
 
 static int fail(qas_ctx* c, int code, const std::string& msg)
@@ -133,7 +129,7 @@ size_t ctx_layout(qas_ctx* c, char* base, double* state)
   const int ndim = c->geo.ndim;
   const long long nd = c->geo.nd;
   const size_t stride = (size_t)((nd + 63) / 64 * 64);
-  const int nprim = ndim == 3 ? 7 : (ndim == 2 ? 6 : 4);
+  const int nprim = ndim == 3 ? 7 : (ndim == 2 ? 6 : 0);
   const int nacc = ndim == 1 ? 0 : (ndim == 2 ? 6 : 10);
   const int nemf = ndim == 3 ? 12 : (ndim == 2 ? 8 : 0);
   const int nedge = ndim == 3 ? 3 : (ndim == 2 ? 1 : 0);
@@ -150,11 +146,9 @@ size_t ctx_layout(qas_ctx* c, char* base, double* state)
       c->U[b][m] = p;
       p += stride;
     }
-  c->vx = p; p += stride;
-  c->vy = p; p += stride;
-  c->vz = p; p += stride;
-  c->pr = p; p += stride;
-  if (ndim >= 2) { c->cx = p; p += stride; c->cy = p; p += stride; }
+  if (ndim >= 2) {  // (the 1D stage keeps its primitives in LDS)
+    for (double** a : {&c->vx, &c->vy, &c->vz, &c->pr, &c->cx, &c->cy}) { *a = p; p += stride; }
+  }
   if (ndim == 3) { c->cz = p; p += stride; }
   for (int k = 0; k < nacc; k++) { c->acc[k] = p; p += stride; }
   for (int k = 0; k < nemf; k++) { c->emf[k] = p; p += stride; }
@@ -368,7 +362,7 @@ extern "C" int qas_cfl_dt(qas_ctx* c, double* dt_out)
   if (!ready(c)) return fail(c, QAS_E_ARG, "qas_cfl_dt: null context");
   if (!c->uploaded) return fail(c, QAS_E_STATE, "qas_cfl_dt: no state uploaded");
   QAS_CHECK(c, launch_cfl(c, c->U[c->cur]));
-  QAS_CHECK(c, launch_cfl_finalize(c, nullptr));
+  QAS_CHECK(c, launch_cfl_finalize(c));
   QAS_CHECK(c, hipMemcpyAsync(c->h_pinned, c->d_dt, sizeof(double), hipMemcpyDeviceToHost, c->stream));
   QAS_CHECK(c, hipStreamSynchronize(c->stream));
   if (dt_out) *dt_out = c->h_pinned[0];
@@ -483,7 +477,7 @@ static int loop_step(qas_ctx* c, int flg, bool hist, bool even)
   if (r) return r;
   if (flg && even) {
     QAS_CHECK(c, launch_cfl(c, c->U[c->cur]));
-    QAS_CHECK(c, launch_cfl_finalize(c, nullptr));
+    QAS_CHECK(c, launch_cfl_finalize(c));
   }
   return QAS_OK;
 }
@@ -538,7 +532,7 @@ extern "C" int qas_run(qas_ctx* c, int nsteps, int flg, double* dt_inout, double
     QAS_CHECK(c, launch_set_dt(c, *dt_inout));
   } else {
     QAS_CHECK(c, launch_cfl(c, c->U[c->cur]));
-    QAS_CHECK(c, launch_cfl_finalize(c, nullptr));
+    QAS_CHECK(c, launch_cfl_finalize(c));
   }
   // the first run of a 2D context picks its launch shape (qas_tune)
   if (!c->tuned && c->g.ndim == 2 && c->prof_mask == 0 && nsteps > 0) {

@@ -97,14 +97,12 @@ __global__ __launch_bounds__(1024) void k_cfl_one(CflArgs a, Geo g, double* dt, 
   }
 }
 
-__global__ __launch_bounds__(256) void k_cfl_final(const double* part, int nb, double* dt, double* hist_slot,
-                                                   double cfl_dr)
+__global__ __launch_bounds__(256) void k_cfl_final(const double* part, int nb, double* dt, double cfl_dr)
 {
-  cfl_final_block(part, nb, dt, hist_slot, cfl_dr);
+  cfl_final_block(part, nb, dt, cfl_dr);
 }
 
 __global__ void k_set_dt(double* dt, double v) { *dt = v; }
-__global__ void k_copy1(const double* src, double* dst) { *dst = *src; }
 // dt history for graph replays: hist[*cnt] = *dt; ++*cnt (one thread)
 __global__ void k_record(const double* dt, double* hist, long long* cnt, long long cap)
 {
@@ -154,23 +152,17 @@ hipError_t launch_cfl(qas_ctx* c, const double* const U[8])
   return hipGetLastError();
 }
 
-hipError_t launch_cfl_finalize(qas_ctx* c, double* hist_slot)
+hipError_t launch_cfl_finalize(qas_ctx* c)
 {
   if (c->cfl_blocks == 0) return hipGetLastError();  // k_cfl_one has set dt
   const double cfl_dr = c->s.cfl * cell_size(c->geo);
-  hipLaunchKernelGGL(k_cfl_final, 1, 256, 0, c->stream, c->d_cflpart, c->cfl_blocks, c->d_dt, hist_slot, cfl_dr);
+  hipLaunchKernelGGL(k_cfl_final, 1, 256, 0, c->stream, c->d_cflpart, c->cfl_blocks, c->d_dt, cfl_dr);
   return hipGetLastError();
 }
 
 hipError_t launch_set_dt(qas_ctx* c, double dt)
 {
   hipLaunchKernelGGL(k_set_dt, 1, 1, 0, c->stream, c->d_dt, dt);
-  return hipGetLastError();
-}
-
-hipError_t launch_record_dt(qas_ctx* c, double* slot)
-{
-  hipLaunchKernelGGL(k_copy1, 1, 1, 0, c->stream, c->d_dt, slot);
   return hipGetLastError();
 }
 

@@ -198,17 +198,12 @@ __device__ __forceinline__ void cfl_block(const CflArgs& a, const Geo& g, int bl
 
 // dt = cfl * dr / max(part[0..nb)); one block of 256 threads.  max is
 // exact and order-independent, so dt equals the reference's serial loop.
-__device__ __forceinline__ void cfl_final_block(const double* part, int nb, double* dt, double* hist_slot,
-                                                double cfl_dr)
+__device__ __forceinline__ void cfl_final_block(const double* part, int nb, double* dt, double cfl_dr)
 {
   double vm = 1.0;
   for (int b = threadIdx.x; b < nb; b += blockDim.x) vm = (part[b] > vm) ? part[b] : vm;
   vm = block_max(vm);
-  if (threadIdx.x == 0) {
-    const double d = cfl_dr / vm;
-    *dt = d;
-    if (hist_slot) *hist_slot = d;
-  }
+  if (threadIdx.x == 0) *dt = cfl_dr / vm;
 }
 
 }  // namespace qas

@@ -191,12 +191,6 @@ __device__ __forceinline__ double load_as(const double* a, long long i)
   return (double)G(reinterpret_cast<const ST*>(a))[i];
 }
 
-template <typename PT>
-__device__ __forceinline__ void store_prim(double* a, long long t, double v)
-{
-  reinterpret_cast<PT*>(a)[t] = (PT)v;
-}
-
 // Ghost-index resolution: bound() writes ghost cells as (factor x) a kept
 // cell of the same array.  Applying x then y then z (bc2d/bc3d order) to a
 // cell gives value = kz*(ky*(kx*f[src])) with the sources below.
@@ -332,7 +326,7 @@ constexpr long long FUSE_MAX = 300LL * 300;
 inline bool fused_emf_ct(const Geo& g) { return g.ndim == 2 && g.nd <= FUSE_MAX; }
 hipError_t launch_bound(qas_ctx* c, double* const f[8], int nvar);
 hipError_t launch_cfl(qas_ctx* c, const double* const U[8]);
-hipError_t launch_cfl_finalize(qas_ctx* c, double* hist_slot);
+hipError_t launch_cfl_finalize(qas_ctx* c);
 hipError_t launch_set_dt(qas_ctx* c, double dt);
 hipError_t launch_record_counted(qas_ctx* c);
 hipError_t launch_zero_counter(qas_ctx* c);

@@ -132,7 +132,7 @@ extern "C" int qas_run_static(const qas_grid* g, const qas_scheme* s, double* d_
     QAS_SCHECK(launch_set_dt(&c, dt));
   } else {
     QAS_SCHECK(launch_cfl(&c, c.U[c.cur]));
-    QAS_SCHECK(launch_cfl_finalize(&c, nullptr));
+    QAS_SCHECK(launch_cfl_finalize(&c));
   }
   QAS_SCHECK(launch_bound(&c, c.U[c.cur], 8));
   for (int k = 1; k <= nsteps; k++) {
@@ -141,7 +141,7 @@ extern "C" int qas_run_static(const qas_grid* g, const qas_scheme* s, double* d_
     if (r) return say(err, errlen, r, "qas_run_static: %s", c.err.c_str());
     if (flg && n % 2 == 0) {
       QAS_SCHECK(launch_cfl(&c, c.U[c.cur]));
-      QAS_SCHECK(launch_cfl_finalize(&c, nullptr));
+      QAS_SCHECK(launch_cfl_finalize(&c));
     }
   }
   // R_K = 1 rotates through the three buffers: bring the state home

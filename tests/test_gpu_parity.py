@@ -273,6 +273,14 @@ def test_1d_stage_and_ghosts_vs_oracle(qas, oracle, n, dn):
     assert np.array_equal(out, ref, equal_nan=True)
 
 
+def test_1d_context_holds_its_states_only(qas):
+    """The 1D stage keeps its primitives in LDS: three states of 8 arrays on
+    the device, and the small words."""
+    n = 100000
+    with qas.Solver((n + 8,), 1.0 / n) as s:
+        assert 24 * 8 * (n + 8) <= s.device_bytes() < 24 * 8 * (n + 8 + 64) + 16384
+
+
 @pytest.mark.parametrize("nsteps", [1, 255, 256, 300])
 def test_history_through_pinned_buffer_or_direct(qas, oracle, nsteps):
     """The dt history comes back with dt in one wait where it fits the pinned
