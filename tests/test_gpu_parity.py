@@ -278,7 +278,7 @@ def test_1d_context_holds_its_states_only(qas):
     the device, and the small words."""
     n = 100000
     with qas.Solver((n + 8,), 1.0 / n) as s:
-        assert 24 * 8 * (n + 8) <= s.device_bytes() < 24 * 8 * (n + 8 + 64) + 16384
+        assert 24 * 8 * (n + 8) <= s.device_bytes < 24 * 8 * (n + 8 + 64) + 16384
 
 
 @pytest.mark.parametrize("nsteps", [1, 255, 256, 300])
