@@ -170,7 +170,7 @@ struct FastOps {
 
 // the operators, for operands of any size
 struct PlainOps {
-  template <typename T> static QAS_HD T raw(T x) { return T(1.0) / x; }
+  template <typename T> static QAS_HD T raw(T x) { return x; }  // (quot divides by x itself)
   template <typename T> static QAS_HD T inv(T x) { return T(1.0) / x; }
   template <typename T> static QAS_HD T quot(T a, T x, T) { return a / x; }
   template <typename T> static QAS_HD T ratio(T a, T x) { return a / x; }

@@ -79,10 +79,7 @@ static double count_riemann()
   CT F[7];
   g_ops = 0;
   riemann<RMN>(L, R, CT(0.5), CT(5.0 / 3.0), CT(-0.01), CT(-0.02), F);
-  // LHLLD as the algorithm states it: a factor 1/2 in each squared speed,
-  // which the body shares between a side's two, and no reciprocal kept for
-  // two quotients (for HLLD the one makes up for the other)
-  return (double)g_ops + (RMN == 2 ? 2 : 0);
+  return (double)g_ops;
 }
 
 template <int ODR>
@@ -185,40 +182,49 @@ extern "C" int qas_kernel_model(const qas_ctx* c, int kid, double* flops, double
     // the stored ones and applies the RK stage sum (2 mul + 2 add).
     const double per_var = d == 0 ? pc.df + 1.0 + (nd3 - 1) + 4.0 : pc.df + 1.0;
     *flops += inter * nupd * per_var;
-    // bytes: 7 stencil arrays + cell-centred normal B + staggered B (read),
-    // 2*ntan face EMF parts (write), accumulators / state
-    double b = cells * (9.0 + 2.0 * ntan);
-    if (nd3 == 1) b = cells * 8.0;
-    if (nd3 == 2 && d == 1) {
-      // the 2D y sweep computes the primitives of every cell itself from the
-      // 8 state arrays and stores 6 of them for the x sweep
-      *flops += cells * (1 + 3 + 5 + 5 + 4 + 2 * pc.fc);
-      b = cells * (8.0 + 6.0 + 2.0 * ntan);
-    }
-    if (d == 0) b += inter * nupd * ((nd3 - 1) + 3.0);  // stored divergences + in, u0 read; out write
-    else b += inter * nupd * 1.0;                        // this sweep's divergence written
+    // The first sweep of a stage (1D: its only launch, x; 2D: y; 3D: z) forms
+    // the primitives of every cell from the 8 state arrays.
+    const bool first = d == nd3 - 1;
+    const int nprim = nd3 == 3 ? 7 : (nd3 == 2 ? 6 : 0);  // stored for the other sweeps
+    if (first) *flops += cells * (1 + 3 + 5 + 5 + 4 + (nd3 >= 2 ? nd3 * pc.fc : 0));
+    // bytes: that sweep reads the state and writes the primitives; another
+    // reads 7 stencil arrays, the cell-centred and the staggered normal B;
+    // each writes 2*ntan face parts
+    double b = cells * ((first ? 8.0 + nprim : 9.0) + 2.0 * ntan);
+    // x: stored divergences, state (read already in 1D) and base of the step
+    // read, the new state written (1D: bx too); the others: their divergence
+    if (d == 0) b += inter * (nd3 == 1 ? 2.0 * nupd + 1.0 : nupd * ((nd3 - 1) + 3.0));
+    else b += inter * nupd * 1.0;
     *bytes = b * 8.0;
     return QAS_OK;
   }
-  if (kid == QAS_K_PRIM) {
-    if (nd3 == 2) return QAS_OK;  // folded into the y sweep
-    *flops = cells * (1 + 3 + 5 + 5 + 4 + (nd3 >= 2 ? nd3 * (pc.fc + 0) : 0));
-    *bytes = cells * 8.0 * (8 + (nd3 >= 2 ? nd3 : 0) + 4);
-    return QAS_OK;
-  }
-  if (kid == QAS_K_EMF) {
+  if (kid == QAS_K_PRIM) return QAS_OK;  // no launch of their own
+  // the corner EMF of a small 2D domain never leaves the CT's launch
+  const bool fused = fused_emf_ct(c->geo);
+  double eflops, ebytes;
+  {
     const double ne = (n[0] - 5) * (nd3 >= 2 ? n[1] - 5 : 1) * (nd3 >= 3 ? n[2] - 5 : 1);
     const double ncomp = nd3 == 3 ? 3 : 1;
     const double part = 4 * pc.lin + 2 + 1 + 2 + 1;  // 4 one-sided interps, (uL+uR)+w(cL+cR), scale
-    *flops = ne * ncomp * (2 * part + 2 + (c->s.ctw ? count_cuct() : 0));
-    *bytes = ne * ncomp * 8.0 * (4 + 1) + (c->s.ctw ? ne * 8.0 * 5 : 0);
+    eflops = ne * ncomp * (2 * part + 2 + (c->s.ctw ? count_cuct() : 0));
+    ebytes = ne * ncomp * 8.0 * (4 + (fused ? 0 : 1)) + (c->s.ctw ? ne * 8.0 * 5 : 0);
+  }
+  if (kid == QAS_K_EMF) {
+    if (fused || nd3 == 1) return QAS_OK;
+    *flops = eflops;
+    *bytes = ebytes;
     return QAS_OK;
   }
   if (kid == QAS_K_CT) {
+    if (nd3 == 1) return QAS_OK;
     const double nf = (n[0] - 7) * (nd3 >= 2 ? n[1] - 7 : 1) * (nd3 >= 3 ? n[2] - 7 : 1);
     const double ncomp = nd3 == 3 ? 3 : 2;
     *flops = nf * ncomp * ((nd3 == 3 ? 2 : 1) * (pc.df + 1) + 1 + 4);
-    *bytes = nf * ncomp * 8.0 * (3 + (nd3 == 3 ? 2 : 1));
+    *bytes = nf * ncomp * 8.0 * (3 + (fused ? 0 : (nd3 == 3 ? 2 : 1)));
+    if (fused) {
+      *flops += eflops;
+      *bytes += ebytes;
+    }
     return QAS_OK;
   }
   return QAS_E_ARG;

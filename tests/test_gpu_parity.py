@@ -281,6 +281,39 @@ def test_1d_context_holds_its_states_only(qas):
         assert 24 * 8 * (n + 8) <= s.device_bytes < 24 * 8 * (n + 8 + 64) + 16384
 
 
+@pytest.mark.parametrize("shape", [(64,), (48, 40), (40, 2500), (16, 18, 20)])
+@pytest.mark.parametrize("rmn", [1, 2])
+def test_work_model_is_of_the_launches(qas, shape, rmn):
+    """qas_kernel_model has work for the kernels a step launches and none for
+    the others; the stage's work does not depend on how it is cut into
+    launches but for the corner EMF's way through memory."""
+    import ctypes as C
+    sh = tuple(m + 8 for m in shape)
+    st = np.zeros((8,) + sh)
+    st[0], st[4], st[7] = 1.0, 0.5, 3.0
+    work = []
+    _say("work model", shape, rmn)
+    with qas.Solver(sh, 0.1, 0.1, 0.1, rmn=rmn) as s:
+        s.upload(st)
+        s.bound()
+        s.sync()
+        s.lib.qas_prof_enable(s.ctx, (1 << 6) - 1, 64)
+        s.step(1e-3)
+        for kid in range(6):
+            ms, n, fl, by = C.c_double(), C.c_longlong(), C.c_double(), C.c_double()
+            assert s.lib.qas_prof_query(s.ctx, kid, C.byref(ms), C.byref(n)) == 0
+            r = s.lib.qas_kernel_model(s.ctx, kid, C.byref(fl), C.byref(by))
+            assert n.value in (0, 3) and (n.value > 0) == (r == 0 and fl.value > 0) == (r == 0 and by.value > 0), kid
+            work.append((n.value, fl.value, by.value) if r == 0 else (0, 0.0, 0.0))
+        s.lib.qas_prof_enable(s.ctx, 0, 0)
+    cells = np.prod(sh, dtype=float)
+    # every launch moves the state or more, and the stage at least 16 arrays
+    assert sum(w[2] for w in work) > 16 * 8 * np.prod(shape) and all(w[2] < 8 * 60 * cells for w in work)
+    pf = (C.c_double * 8)()
+    s.lib.qas_point_flops(rmn, 4, pf)
+    assert sum(w[1] for w in work) > len(shape) * np.prod(shape) * (min(pf[0], pf[1]) + pf[2])
+
+
 @pytest.mark.parametrize("nsteps", [1, 255, 256, 300])
 def test_history_through_pinned_buffer_or_direct(qas, oracle, nsteps):
     """The dt history comes back with dt in one wait where it fits the pinned
