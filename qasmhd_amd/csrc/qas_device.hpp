@@ -716,8 +716,7 @@ QAS_HD void flux_hlld_family(const bool lowdiss, const T* L, const T* R, T bnc, 
   // so the root of the larger square is the larger root.  HLLD compares the
   // roots (LHLLD the squares): a negative right square, of a negative density,
   // must come through as its NaN does
-  T cf2 = tmax(cfl2, cfr2);
-  if (!lowdiss) cf2 = cfr2 < T(0) ? cfr2 : cf2;
+  const T cf2 = (cfl2 >= cfr2) & (lowdiss | (cfr2 >= T(0))) ? cfl2 : cfr2;
   const T cmax = O::root(T(0.5) * cf2);
   const T sl = tmin(T(0.0), tmin(vnl, vnr) - cmax);
   const T sr = tmax(T(0.0), tmax(vnl, vnr) + cmax);
