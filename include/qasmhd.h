@@ -57,7 +57,10 @@ typedef struct {
   int dn[3][8];     /* boundary flags dnxs/dnys/dnzs: 0 periodic, +-1
                        Neumann/Dirichlet, +-2 open/zero-fix                 */
   int st[3][8];     /* staggering flags stxs/stys/stzs (bx:x, by:y, bz:z = 1) */
-  int precision;    /* 0 = FP64 (bit-identical to the reference),
+  int precision;    /* 0 = FP64 (bit-identical to the reference; for densities
+                           past 1e+-302 and speeds past 1e+-76, whose fourth
+                           powers leave the exponent range, up to rounding
+                           and the reference's own underflow),
                        1 = mixed (FP32 reconstruction and fluxes; FP64 state,
                            RK stage sum and pressure recovery),
                        2 = FP64 with fused multiply-adds in the sweeps (same

@@ -50,7 +50,7 @@ struct StagePtrs {
 
 // The primitive scratch as the sweeps read it: element type PT = the
 // reconstruction precision (double: FP64 path; float: mixed path, where the
-// prim kernels round the FP64 primitives once on store).
+// first sweep rounds the FP64 primitives once on store).
 template <typename PT>
 struct PrimView {
   const PT *vx, *vy, *vz, *pr, *cx, *cy, *cz;

@@ -1,7 +1,8 @@
 // qas_kernels2d.hip -- one SSP-RK stage of the 2D ideal-MHD step on gfx950.
 //
 // Replaces the stage body of MHD2D::ideal (2D/SERIAL/OTvortex/
-// mhd2d_solve.cpp:44-386).  A stage is four launches:
+// mhd2d_solve.cpp:44-386).  A stage is four launches, three for domains of up to
+// 300^2 cells (emf2d and ct2d in one, k_emfct2d):
 //   sweep<Y> cell-centred B and primitives of its LDS tile from the state
 //            (stored for the x sweep)                        (:51-89)
 //            then characteristic WCNS + Riemann flux per y face, for every
@@ -15,8 +16,8 @@
 //   ct2d     staggered bx, by update                        (:359-380)
 //            and the bound() of the stage output             (:384-385)
 // A lane of a sweep reconstructs one cell; neighbour states and fluxes move
-// between lanes (qas_sweep2d.hpp).  Everything runs in FP64 with the reference's operation
-// order (the library is built with -ffp-contract=off).
+// between lanes (qas_sweep2d.hpp).  Everything runs in FP64 with the reference's
+// operation order (the library is built with -ffp-contract=off).
 #include "qas_device.hpp"
 #include "qas_internal.hpp"
 #include "qas_stage2d.hpp"

@@ -32,11 +32,10 @@ namespace qas {
 // for Ez): the parts interpolated along it sit in 6-point register windows and
 // the two cells behind are carried, so each is read once.  Per edge the
 // operations and their order are the reference's.
-// One thread for all three components needed 256 VGPRs (2 wavefronts per SIMD)
-// and ran at 2.4 TB/s, waiting on its loads: 188 us at 128^3 (FP64), 382 at
-// 200^3 (mixed); one component per thread 147 and 335 (116 VGPRs).  At
-// 512^3, where Ez's run no longer finds the cells of Ex's and Ey's in the L2, it
-// takes 8.5 ms against 7.6 (FP64; the whole stage 47.3 against 51.6).
+// One thread for all three components takes 256 VGPRs (2 wavefronts per SIMD)
+// and waits on its loads where there are few columns: 182 us at 128^3 (FP64),
+// 383 at 200^3 (mixed); one component per thread 147 and 336 (116 VGPRs).
+// Large domains: k_emf3d_z.
 // FT: the sweep precision, the type of the face parts, of the velocities (the
 // primitives the z sweep stored) and of the edge EMFs; arithmetic is FP64.
 template <int ODR>

@@ -2,8 +2,8 @@
 //
 // Reconstruction (characteristic projection + WCNS), the Riemann solver and
 // the B-flux face states run in FP32; the conserved state, the primitive /
-// pressure recovery (prim kernels), the flux differencing, the RK stage sum
-// and the CT update stay FP64.  This translation unit is compiled with
+// pressure recovery (the first sweep's staging), the flux differencing, the RK
+// stage sum and the CT update stay FP64.  This translation unit is compiled with
 // -fno-hip-fp32-correctly-rounded-divide-sqrt (FP32 divide and sqrt by the
 // hardware reciprocal / square-root estimates with their refinement) and
 // with FMA contraction; its error against the FP64 path is measured, not

@@ -75,7 +75,7 @@ __device__ __forceinline__ Prim2d prim2d_cell(const StagePtrs& p, const Geo& g, 
 }
 
 // velocity component of cell c from the state: the same expression as the
-// prim kernel (m * (1/ro)), so the FP64 value is bit-identical to it
+// first sweep's primitives (m * (1/ro)), so the FP64 value is bit-identical to it
 __device__ __forceinline__ double vel(const StagePtrs& p, int comp, long long c)
 {
   return p.in[1 + comp][c] * FastOps::inv(p.in[0][c]);

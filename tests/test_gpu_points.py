@@ -195,3 +195,19 @@ def test_flux_of_broken_states(pts, oracle, rmn, side, var):
         q[s, :, var] *= -1.0
     out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
     assert _eq_nan(out, ref)
+
+
+@pytest.mark.parametrize("rmn", [0, 1, 2, 3])
+def test_flux_to_the_ends_of_its_range(pts, oracle, rmn):
+    """Speeds of 1e-76 to 1e76 (their fourth powers are normal numbers) and
+    densities of 1e-302 to 1e302: the oracle's values."""
+    print("case: flux, ends of the range, rmn", rmn, flush=True)
+    rng = np.random.default_rng(70 + rmn)
+    n = 20000
+    for d, v in [(1.0, 10.0 ** k) for k in (-76, -60, 60, 76)] + [(10.0 ** k, 1.0) for k in (-302, -290, 290, 302)]:
+        q = rng.uniform(0.5, 2.0, (2, n, 7)) * np.where(np.arange(7) % 6 == 0, 1.0, rng.choice([-1.0, 1.0], (2, n, 7)))
+        b = np.sqrt(d) * v
+        q *= np.array([d, v, v, v, b, b, d * v * v])
+        bn, dv = rng.uniform(-2.0, 2.0, n) * b, rng.uniform(-0.2, 0.2, (n, 2)) * v
+        out, ref = pts.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv), oracle.flux(rmn, q[0], q[1], bn, 5.0 / 3.0, dv)
+        assert np.isfinite(ref).any() and _eq_nan(out, ref), (d, v)
